@@ -60,12 +60,39 @@ BPMH_DEV double d_sub(double a, double b) {
   return a - b;
 }
 
-// cos/sin of a float32 angle, evaluated in float64 and rounded to float32:
-// bit-reproducible against a float64 libm for all but ~2^-28 of inputs.
+// cos/sin of a float32 angle, evaluated in float64 and rounded to float32.
+// The angle less its nearest multiple of pi/2 (two FMAs with pi/2 split into
+// two float64 parts, exact to 2^-54 for |x| < 2^31) goes through the Taylor
+// series of sin to r^13 and cos to r^14 on [-pi/4, pi/4]; the first omitted
+// terms are below 2.1e-14 and 1.1e-15 (no rounded result differed from the
+// exact values' over 4 million arguments up to 2000).  27 float64 operations
+// and no branch, against the library's sincos with its reduction for
+// arguments of any size: weighted pass B at 1024^2, whose time after the mean
+// is known is this evaluation, 13.64 -> 13.24 us (kernel trace).
 BPMH_DEV float2 sincos_f32_via_f64(float ph) {
-  double s, c;
-  sincos((double)ph, &s, &c);
-  return make_float2((float)c, (float)s);
+  const double x = (double)ph;
+  const double n = rint(x * 0.63661977236758134308);       // 2/pi
+  double r = fma(-n, 1.57079632679489655800, x);            // pi/2, high part
+  r = fma(-n, 6.12323399573676603587e-17, r);               // low part
+  const double r2 = r * r;
+  double s = fma(r2, 1.60590438368216145994e-10, -2.50521083854417187751e-8);  // 1/13!, -1/11!
+  s = fma(r2, s, 2.75573192239858906526e-6);                // 1/9!
+  s = fma(r2, s, -1.98412698412698412698e-4);               // -1/7!
+  s = fma(r2, s, 8.33333333333333333333e-3);                // 1/5!
+  s = fma(r2, s, -1.66666666666666666667e-1);               // -1/3!
+  s = fma(r * r2, s, r);
+  double c = fma(r2, -1.14707455977297247139e-11, 2.08767569878680989792e-9);  // -1/14!, 1/12!
+  c = fma(r2, c, -2.75573192239858906526e-7);               // -1/10!
+  c = fma(r2, c, 2.48015873015873015873e-5);                // 1/8!
+  c = fma(r2, c, -1.38888888888888888889e-3);               // -1/6!
+  c = fma(r2, c, 4.16666666666666666667e-2);                // 1/4!
+  c = fma(r2, c, -0.5);
+  c = fma(r2, c, 1.0);
+  const float sf = (float)s, cf = (float)c;
+  // quarter turns: n mod 4
+  const int q = (int)(n - 4. * floor(n * 0.25));
+  const float a = (q & 1) ? sf : cf, b = (q & 1) ? cf : sf;
+  return make_float2((q == 1 || q == 2) ? -a : a, (q & 2) ? -b : b);
 }
 
 // sin and cos of a float32 angle.  For |x| <= pi/4 (every phase screen of a
