@@ -14,9 +14,7 @@
 // default mean_mode "weighted" of bpm_3d needs the k-space reduction of
 // bpm_3d.py:302-303 before H, so its column pass is split in two (A: FFT_y
 // and per-column partial sums; B: H(n0+dn0) and IFFT_y).
-#include "common.hpp"
-#include "fft.hpp"
-#include "bpm_hip.h"
+#include "loop.hpp"
 
 #include <cmath>
 #include <cstdint>
@@ -24,10 +22,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
-#include <type_traits>
 #include <vector>
-
-using namespace bpmfft;
 
 // ----------------------------------------------------------------------------
 // error reporting
@@ -53,252 +48,8 @@ extern "C" const char* bpmh_last_error(void) { return g_err.c_str(); }
 extern "C" int bpmh_version(void) { return BPMH_VERSION; }
 
 // ----------------------------------------------------------------------------
-// per-size launch configurations: variant V in {0,1,2} scales the default
-// number of lines (rows) or columns per work-group by 1/2, 1, 2, clamped to
-// 1..16 lines, 1024 threads and 128 KiB of LDS (gfx950 has 160 KiB per CU);
-// the autotuner picks V per size.
-// ----------------------------------------------------------------------------
-constexpr int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
-constexpr int pow2floor(int v) { return v < 2 ? 1 : 2 * pow2floor(v / 2); }
-constexpr int scale_v(int base, int V) { return V == 0 ? base / 2 : (V == 1 ? base : base * 2); }
-
-// Elements per thread of a line.  Rows: 4 up to N = 1024 (twice the
-// wavefronts of E = 8 for the same data, so loads, transforms and stores of
-// different wavefronts overlap better; measured 5-13 % faster per z-step at
-// 64^2..1024^2, batch 1), 8 above.  Columns: 8 (4-column tiles of 8-element
-// threads; E = 4 measured slower at 1024^2, also with 4-column tiles of
-// 1024 threads, and at 256^2..512^2 in batches).
-constexpr int row_e(int n) { return n <= 1024 ? 4 : 8; }
-constexpr int col_e(int n) { return n <= 32 ? 4 : 8; }
-// The other radix schedule of a size, which the autotuner times against the
-// default: 8 elements per thread instead of 4 (when the line still holds two
-// radix-8 stages, N >= 64), or 4 instead of 8.  ealt selects it.
-constexpr int alt_e(int e, int n) { return e == 4 ? (n >= 64 ? 8 : 4) : 4; }
-constexpr int row_e_of(int n, int ealt) { return ealt ? alt_e(row_e(n), n) : row_e(n); }
-constexpr int col_e_of(int n, int ealt) { return ealt ? alt_e(col_e(n), n) : col_e(n); }
-// Variant numbers: row variant = V + 3*ealt (V = 0, 1, 2), column variant =
-// V + 5*ealt (V = 0..4).
-constexpr int kRowShapes = 3, kColShapes = 5;
-#define BPMH_MAX_GROUPS 16
-
-
-template <int N, int E_>
-struct Base {
-  static constexpr int E = E_;
-  static constexpr int T = N / E;
-  // LDS (layouts of fft.hpp): a row line is N float2 in the swizzled
-  // exchange layout (8 more when lines of fewer than 16 threads share a
-  // 16-lane group, so those lines start in different banks).  Column tiles
-  // of 4 or more columns use the swizzled layout for C = COLS lines per
-  // 16-lane group, lines N + 16/COLS apart; narrower tiles keep lines padded
-  // one per 32 and 9 float2 longer (the swizzle measured slower there).
-  // COL_LINE, the padded length, bounds both.
-  static constexpr int ROW_LINE = N + (T < 16 ? 8 : 0);
-  static constexpr int COL_SH = 5;
-  static constexpr int COL_LINE = N + (N >> COL_SH) + 9;  // float2 per column line
-  static constexpr int LDS_LINE = COL_LINE * 8;        // bytes per column line
-};
-
-template <int N, int V, int E_ = row_e(N)>
-struct RowCfg : Base<N, E_> {
-  using Base<N, E_>::T;
-  static constexpr int L0 = clampi(256 / T, 1, 16);
-  // at least one full wavefront per work-group (the cross-lane reductions
-  // use all 64 lanes), at most 16 lines and 1024 threads
-  static constexpr int LMIN = 64 / T < 1 ? 1 : 64 / T;
-  static constexpr int LINES =
-      clampi(clampi(scale_v(L0, V), LMIN, 16), 1, (1024 / T) < 1 ? 1 : 1024 / T);
-  static constexpr int THREADS = LINES * T;
-};
-
-template <int N, int V, int E_ = col_e(N)>
-struct ColCfg : Base<N, E_> {
-  using Base<N, E_>::T;
-  using Base<N, E_>::LDS_LINE;
-  static constexpr int C0 = N >= 4096 ? 1 : clampi(512 / T, 2, 16);
-  static constexpr int CMAX0 = 131072 / LDS_LINE < 1 ? 1 : 131072 / LDS_LINE;
-  // <= 512 threads with 8 elements per thread (1024 spilled), <= 1024 with 4
-  static constexpr int TMAX = (E_ <= 4 ? 1024 : 512) / T < 1 ? 1 : (E_ <= 4 ? 1024 : 512) / T;
-  static constexpr int CMAX = pow2floor(clampi(CMAX0 < TMAX ? CMAX0 : TMAX, 1, 16));
-  static constexpr int CMIN = 64 / T < 1 ? 1 : 64 / T;  // >= one full wavefront
-  // V = 3: the work-group of V = 0 with P = 2 adjacent columns per thread
-  // (tiles twice as wide), so a row of a column pair is one 16-byte load and
-  // store.  V = 4: the same with each column's loads and stores issued
-  // separately (8-byte accesses), the first column's loads first, so its
-  // transform can start while the second column's loads are in flight.
-  // Used for columns of 256-1024 points (where they were measured);
-  // elsewhere they are V = 0.
-  static constexpr bool PAIRED = (V == 3 || V == 4) && N >= 256 && N <= 1024;
-  static constexpr int P = PAIRED ? 2 : 1;
-  static constexpr bool SPLIT = PAIRED && V == 4;
-  static constexpr int LC = clampi(scale_v(C0, V >= 3 ? 0 : V), CMIN, CMAX);  // lane columns
-  static constexpr int COLS = LC * P;
-  static constexpr int THREADS = LC * T;
-};
-
-// ----------------------------------------------------------------------------
-// device helpers
-// ----------------------------------------------------------------------------
-BPMH_DEV float2 load_dn(const void* dn, int kind, size_t idx) {
-  if (kind == BPMH_DN_F32) return make_float2(((const float*)dn)[idx], 0.f);
-  if (kind == BPMH_DN_F16) return make_float2(__half2float(((const __half*)dn)[idx]), 0.f);
-  return ((const float2*)dn)[idx];
-}
-
-// FFTFREQ(i,N,d) of bpm_3d_kernels.cl:6 in float32
-BPMH_DEV float fftfreq_f32(int i, int N, float d) {
-  const int half = (N - 1) / 2 + 1;
-  const float num = (i < half) ? (float)i : (float)((i - half) - N / 2);
-  return f_div(f_div(num, (float)N), d);
-}
-
-BPMH_DEV float kcomp2_f32(int i, int N, float d) {
-  const float k = f_mul(2.f * BPMH_PI_F, fftfreq_f32(i, N, d));
-  return f_mul(k, k);
-}
-
-// H for one (kx^2, ky^2) with a = ((n*n)*k0)*k0, as compute_propagator
-// (bpm_3d_kernels.cl:419-430): (tmp>=0) * exp(-i dz sqrt(tmp)).
-BPMH_DEV float2 prop_f32(float kx2, float ky2, float a, float dz) {
-  const float tmp = f_sub(f_sub(a, kx2), ky2);
-  const float h0 = tmp < 0.f ? 0.f : __fsqrt_rn(tmp);
-  const float2 cs = sincos_f32_via_f64(f_mul(-dz, h0));
-  return tmp >= 0.f ? cs : make_float2(0.f, 0.f);
-}
-
-BPMH_DEV float n_term_f32(float n, float k0) { return f_mul(f_mul(f_mul(n, n), k0), k0); }
-
-// prop_f32 (the same operations, so the same H) that also returns
-// beta = sqrt(a - kx^2 - ky^2), 0 where the component does not propagate
-// (H = 0 there, and its derivative with respect to dn0 is taken as 0).
-BPMH_DEV float2 prop_f32_beta(float kx2, float ky2, float a, float dz, float* beta) {
-  const float tmp = f_sub(f_sub(a, kx2), ky2);
-  const float h0 = tmp < 0.f ? 0.f : __fsqrt_rn(tmp);
-  const float2 cs = sincos_f32_via_f64(f_mul(-dz, h0));
-  *beta = tmp > 0.f ? h0 : 0.f;
-  return tmp >= 0.f ? cs : make_float2(0.f, 0.f);
-}
-
-// Weighted mean (bpm_3d.py:149-159,302-303): dn0 = dn_sum/u_sum over the nx
-// per-column partials of item b (x = dn part, y = u part) that column pass A
-// wrote.  Column pass B forms it once per work-group: lane p of the first
-// wavefront sums partials p, p+64, ... and an xor butterfly completes the
-// sum (a fixed order, so every work-group gets the same bits); the result is
-// broadcast through LDS, and the work-group of tile 0 stores it for the row
-// pass.  The kernel boundary after pass A orders the partials' stores before
-// these loads.
-// slot[0] receives dn0, slot[1] the weight sum sum|U| (the adjoint needs it).
-BPMH_DEV float weighted_dn0_group(const float2* __restrict__ wp, int nparts, float* slot) {
-  if (threadIdx.x < 64) {
-    const int lane = threadIdx.x;
-    float sd = 0.f, su = 0.f;
-    for (int p = lane; p < nparts; p += 64) {
-      const float2 v = wp[p];
-      sd += v.x;
-      su += v.y;
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      sd += __shfl_xor(sd, o, 64);
-      su += __shfl_xor(su, o, 64);
-    }
-    if (lane == 0) {
-      slot[0] = sd / su;
-      slot[1] = su;
-    }
-  }
-  __syncthreads();
-  return slot[0];
-}
-
-// Sum of n1 floats at p1 and of n2 floats at p2 by the first wavefront in a
-// fixed order (lane l takes elements l, l+64, ..., then an xor butterfly),
-// so every work-group of an item gets the same bits; returned to all
-// threads through slot[0..1].
-BPMH_DEV float2 group_sum_pair(const float* __restrict__ p1, int n1, const float* __restrict__ p2,
-                               int n2, float* slot) {
-  if (threadIdx.x < 64) {
-    const int lane = threadIdx.x;
-    float s1 = 0.f, s2 = 0.f;
-    for (int i = lane; i < n1; i += 64) s1 += p1[i];
-    for (int i = lane; i < n2; i += 64) s2 += p2[i];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      s1 += __shfl_xor(s1, o, 64);
-      s2 += __shfl_xor(s2, o, 64);
-    }
-    if (lane == 0) {
-      slot[0] = s1;
-      slot[1] = s2;
-    }
-  }
-  __syncthreads();
-  return make_float2(slot[0], slot[1]);
-}
-
-// Sum over the T threads of each column of a tile, in a fixed binary-tree
-// order that depends only on T (not on how many columns share the
-// work-group), so per-column partial sums are identical for every launch
-// shape.  Uses the tile's LDS lines as scratch; returns the sum in t == 0.
-template <int T>
-BPMH_DEV float2 column_sum2(float2 v, float2* __restrict__ col_lds, int t) {
-  __syncthreads();  // the FFT's last reads of col_lds are done
-  col_lds[t] = v;
-  __syncthreads();
-#pragma unroll
-  for (int s = T / 2; s > 0; s >>= 1) {
-    if (t < s) col_lds[t] = c_add(col_lds[t], col_lds[t + s]);
-    __syncthreads();
-  }
-  return col_lds[0];
-}
-
-// ----------------------------------------------------------------------------
 // row pass
 // ----------------------------------------------------------------------------
-struct RowArgs {
-  float2* plane;           // (rows = batch*ny, nx)
-  const float2* tw;        // stage-major twiddles of the nx-point transform
-  const void* dn;          // (nz, ny, nx) per batch item, kind dn_kind
-  long long dn_bstride;    // elements between batch items' (or groups') dn (0: shared)
-  // ragged batch: items [gend[g-1], gend[g]) read dn volume g; ngroups = 0:
-  // item b reads volume b
-  int ngroups;
-  int gend[BPMH_MAX_GROUPS];
-  int dn_kind;
-  int ny, nz, z;
-  float unit_k;            // float32(k0*dz)
-  float inv_n;             // 1/(nx*ny)
-  int absorb;
-  int dn0_mode;            // BPMH_MEAN_*: 0 none, 1 per-plane array, 2 weighted
-  const float* dn0_arr;    // simple mode: float32 dn0 per plane
-  const float* dn0_item;   // weighted: dn0 of this step per item (column pass A)
-  float2* out_field;       // (batch, nz, ny, nx) or null
-  float* out_intens;       // (batch, nz, ny, nx) or null
-  float* acc;              // (batch, ny, nx) or null: sum_z |u_z|^2
-  int acc_init;
-  int inverse;             // input is F_x u: inverse FFT first
-  int screen;              // apply dn[z] screen
-  int fwd_items;           // items b < fwd_items get the forward FFT_x before storing
-  // adjoint step: v is the gradient G_z (torch convention, 2 dL/du*); the
-  // row pass writes unit_k*Im(conj(G_z) u_z) per item and multiplies by the
-  // conjugate screen
-  int adjoint;
-  const float2* useg;      // forward planes of the segment (batch, nseg, ny, nx)
-  long long useg_bstride;  // elements between items in useg
-  int useg_z;              // plane of z inside the segment
-  float* gitem;            // (batch, ny, nx) per-item gradient of dn[z] (2 floats per voxel for complex dn)
-};
-
-// dn volume of item b: b itself, or in a ragged batch the group holding b
-// (a few scalar compares; b is uniform over a work-group).
-BPMH_DEV int dn_volume(const RowArgs& a, int b) {
-  if (a.ngroups == 0) return b;
-  int g = 0;
-  while (g + 1 < a.ngroups && b >= a.gend[g]) ++g;
-  return g;
-}
-
 template <int NX, int V, int EE>
 __global__ void __launch_bounds__((RowCfg<NX, V, EE>::THREADS))
 k_row(RowArgs a) {
@@ -352,62 +103,10 @@ k_row(RowArgs a) {
     float dn0 = 0.f;
     if (a.dn0_mode == BPMH_MEAN_SIMPLE) dn0 = a.dn0_arr[a.z];
     else if (a.dn0_mode == BPMH_MEAN_WEIGHTED) dn0 = a.dn0_item[b];
-    const int disty = min(a.ny - y - 1, y);
-#pragma unroll
-    for (int m = 0; m < E; ++m) {
-      const int x = t + m * T;
-      if (a.dn_kind == BPMH_DN_C64) {
-        // cexp((0,-k)*(dn - dn0)) = e^{k Im} (cos(-k Re), sin(-k Re)), no taper
-        const float re = f_mul(a.unit_k, d[m].y);
-        const float im = f_mul(-a.unit_k, f_sub(d[m].x, dn0));
-        float s, c;
-        sincos_fast(im, &s, &c);
-        const float mag = expf(re);
-        if (a.adjoint) {
-          // u = s v with s = e^{k Im dn} e^{-i k Re dn}: dL/dRe dn = k Im(conj(G) u),
-          // dL/dIm dn = k Re(conj(G) u), and G_v = conj(s) G
-          const float2 w = make_float2(v[m].x * ua[m].x + v[m].y * ua[m].y,
-                                       v[m].x * ua[m].y - v[m].y * ua[m].x);
-          reinterpret_cast<float2*>(a.gitem)[((size_t)b * a.ny + y) * NX + x] =
-              make_float2(a.unit_k * w.y, a.unit_k * w.x);
-          v[m] = c_mulc(v[m], make_float2(mag * c, mag * s));
-        } else {
-          v[m] = c_mul(v[m], make_float2(mag * c, mag * s));
-        }
-      } else {
-        const float ph = f_mul(-a.unit_k, f_sub(d[m].x, dn0));
-        float s, c;
-        sincos_fast(ph, &s, &c);
-        float2 r;
-        if (a.adjoint) {
-          a.gitem[((size_t)b * a.ny + y) * NX + x] = a.unit_k * (v[m].x * ua[m].y - v[m].y * ua[m].x);
-          r = c_mulc(v[m], make_float2(c, s));
-        } else {
-          r = c_mul(v[m], make_float2(c, s));
-        }
-        if (a.absorb > 0) {  // uniform: no taper work at all without one
-          const int dist = min(min(NX - x - 1, x), disty);
-          if (dist < a.absorb) {
-            const float arg = f_div(f_mul(BPMH_PI_F, (float)dist), (float)a.absorb);
-            const float tp = f_mul(0.5f, f_sub(1.f, (float)cos((double)arg)));
-            r = make_float2(r.x * tp, r.y * tp);
-          }
-        }
-        v[m] = r;
-      }
-    }
+    row_screen<NX, E, true>(a, b, y, t, dn0, d, ua, v);
   }
 
-  if (a.out_field) {
-    float2* o = a.out_field + ((size_t)b * a.nz + a.z) * a.ny * NX + plane_off;
-#pragma unroll
-    for (int m = 0; m < E; ++m) st_stream(o + t + m * T, v[m]);
-  }
-  if (a.out_intens) {
-    float* o = a.out_intens + ((size_t)b * a.nz + a.z) * a.ny * NX + plane_off;
-#pragma unroll
-    for (int m = 0; m < E; ++m) st_stream(o + t + m * T, v[m].x * v[m].x + v[m].y * v[m].y);
-  }
+  row_outputs<NX, E>(a, a.z, b, plane_off, t, v);
   if (acc_row) {
 #pragma unroll
     for (int m = 0; m < E; ++m) {
@@ -424,46 +123,6 @@ k_row(RowArgs a) {
 // ----------------------------------------------------------------------------
 // column pass
 // ----------------------------------------------------------------------------
-struct ColArgs {
-  float2* plane;           // (batch, ny, nx)
-  const float2* tw;        // stage-major twiddles of the ny-point transform
-  int nx, nz, z;
-  int hmode;               // 0: table H, 1: formula with n_eff[z], 2: formula with n0+weighted dn0
-  const float2* H;         // (ny, nx)
-  const float* n_eff;      // per plane, float32
-  float n0, k0, dx, dy, dz;
-  const void* dn;          // weighted: slice 0 of each item's dn is the weight
-  long long dn_bstride;
-  int dn_kind;
-  float2* wpart;           // weighted per-column partials (batch, nx)
-  float* dn0_item;         // weighted: dn0 per item, stored by pass B for the row pass
-  const float* sw;         // scattering weights (ny, nx) or null
-  const float* gw;
-  const float2* pw;        // plane-wave DC per plane (nz)
-  float2* spart;           // scattering per-column partials (batch, nz, nx)
-  int conj_h;              // adjoint: multiply by conj(H)
-  // forward recorded for the adjoint (null: nothing recorded): PHASE 1, and
-  // PHASE 0 before H, also store U = F u of this step (item stride
-  // kout_bstride); PHASE 2 stores this step's dn0 and sum|U| per item
-  float2* kout;
-  long long kout_bstride;
-  float* rec_c;
-  float* rec_w;
-  // weighted adjoint (PHASE 3, 4) of the step whose forward k-space plane is
-  // U (uk, item stride uk_bstride) with dn0 c = cz[b] and sum|U| = wz[b]
-  const float2* uk;
-  long long uk_bstride;
-  const float* cz;
-  const float* wz;
-  float* s2part;           // (batch, nx): per column sum Im(conj(X) H U) / beta
-  const float* s1part;     // (batch, ny): per row sum of the screen gradient
-  float* gd_item;          // (batch, ny, nx): += dL/d(weight slice) per item
-  // simple mean (PHASE 3, 4): dn0 = mean(dn[z]) does not depend on the
-  // field: n = n_eff[z], no |U| term, and PHASE 4 stores dL/ddn0 per item
-  int simple;
-  float* cg_out;
-};
-
 // PHASE 0: FFT_y, H, IFFT_y.  PHASE 1: FFT_y, weighted partials, store.
 // PHASE 2: weighted dn0, H(n0+dn0), IFFT_y.
 // Adjoint of a weighted step (X = F G_v, the k-space gradient):
@@ -619,16 +278,11 @@ k_col(ColArgs a) {
     float2* line = lds[q * LC + c];
     if constexpr (PHASE == 1) {
       const size_t s0 = (size_t)b * a.dn_bstride;
-      float2 acc = make_float2(0.f, 0.f);
+      float d[E];
 #pragma unroll
-      for (int m = 0; m < E; ++m) {
-        const int ky = t + m * T;
-        const float au = hypotf(v[q][m].x, v[q][m].y);
-        const float d = a.dn ? load_dn(a.dn, a.dn_kind, s0 + (size_t)ky * a.nx + x).x : 0.f;
-        acc.x += au * d;
-        acc.y += au;
-      }
-      acc = column_sum2<T>(acc, line, t);
+      for (int m = 0; m < E; ++m)
+        d[m] = a.dn ? load_dn(a.dn, a.dn_kind, s0 + (size_t)(t + m * T) * a.nx + x).x : 0.f;
+      const float2 acc = col_weight_sums<NY, E>(v[q], d, t, line);
       if (t == 0) a.wpart[(size_t)b * a.nx + x] = acc;
     } else if constexpr (PHASE == 3) {
       // dH/ddn0 = H * (-i dz (n0+dn0) k0^2 / beta): collect Im(conj(X) H U)/beta
@@ -681,42 +335,19 @@ k_col(ColArgs a) {
       }
       if constexpr (PHASE == 2 || PHASE == 4 || PHASE == 5) {
         // H(n0 + dn0) (weighted pass B, its adjoint) or H(n_eff[z]) (simple
-        // mean, its adjoint) on the fly for every row.  H(ky) == H(NY - ky)
-        // bit for bit (kcomp2_f32 of both rows is the same float), and the
-        // rows of thread t mirror those of thread T - t (element m <->
-        // E-1-m; thread 0 mirrors its own, m <-> E-m, and holds row NY/2
-        // alone), so each thread evaluates its first E/2 rows (thread 0 also
-        // row NY/2) and takes the others from its partner through the
-        // column's LDS line (free before the inverse transform).
+        // mean, its adjoint) on the fly for every row
         float2 h[E];
-#pragma unroll
-        for (int m = 0; m < E / 2; ++m)
-          h[m] = prop_f32(kx2, kcomp2_f32(t + m * T, NY, a.dy), an, a.dz);
-        if (t == 0) h[E / 2] = prop_f32(kx2, kcomp2_f32(NY / 2, NY, a.dy), an, a.dz);
-        __syncthreads();  // earlier users of the line are done with it
-#pragma unroll
-        for (int m = 0; m < E / 2; ++m) line[m * T + t] = h[m];
-        __syncthreads();
-        const int pt = T - t;
-#pragma unroll
-        for (int m = E / 2; m < E; ++m) {
-          if (t == 0) {
-            if (m > E / 2) h[m] = h[E - m];
-          } else {
-            h[m] = line[(E - 1 - m) * T + pt];
-          }
-        }
-        __syncthreads();  // before the line is written again
+        col_h_fly<NY, E>(kx2, an, a.dy, a.dz, t, line, h);
 #pragma unroll
         for (int m = 0; m < E; ++m)
-          v[q][m] = a.conj_h ? c_mulc(v[q][m], h[m]) : c_mul(v[q][m], h[m]);
+          v[q][m] = c_mul_fused(v[q][m], make_float2(h[m].x, a.conj_h ? -h[m].y : h[m].y));
       } else {
 #pragma unroll
         for (int m = 0; m < E; ++m) {
           const int ky = t + m * T;
           const float2 h =
               (a.hmode == 0) ? hv[q][m] : prop_f32(kx2, kcomp2_f32(ky, NY, a.dy), an, a.dz);
-          v[q][m] = a.conj_h ? c_mulc(v[q][m], h) : c_mul(v[q][m], h);
+          v[q][m] = c_mul_fused(v[q][m], make_float2(h.x, a.conj_h ? -h.y : h.y));
         }
       }
       if (PHASE == 4 && !a.simple) {
@@ -736,26 +367,7 @@ k_col(ColArgs a) {
           gd[(size_t)ky * a.nx] += cgrad * au * inv_w;
         }
       }
-      if (a.sw) {
-        // scattering reductions of bpm_3d.py:243-247,335-341 on the k-space
-        // plane after H: sum w |U - delta_{k,0} plain|^2
-        float2 acc = make_float2(0.f, 0.f);
-        const float2 pl = a.pw[a.z];
-#pragma unroll
-        for (int m = 0; m < E; ++m) {
-          const int ky = t + m * T;
-          float2 f = v[q][m];
-          if (ky == 0 && x == 0) f = c_sub(f, pl);
-          const float af = hypotf(f.x, f.y);
-          const float a2 = af * af;
-          const size_t k = (size_t)ky * a.nx + x;
-          acc.x += a.sw[k] * a2;
-          acc.y += a.gw[k] * a2;
-        }
-        acc = column_sum2<T>(acc, line, t);
-        if (t == 0) a.spart[((size_t)b * a.nz + a.z) * a.nx + x] = acc;
-        __syncthreads();  // the line is the inverse transform's exchange buffer
-      }
+      if (a.sw) col_scatter<NY, E>(a, a.z, b, x, t, line, v[q]);
     }
   }
   if constexpr (PHASE == 1) {
@@ -881,6 +493,7 @@ struct bpmh_plan_s {
   hipStream_t cap_stream;
   std::vector<GraphEntry> graphs;
   unsigned long long graph_clock;
+  int loop_mode;                // bpmh_plan_set_loop
 };
 
 // Wait for an entry's latest replay, then release it.
@@ -977,6 +590,11 @@ static void make_stage_twiddles(int N, int E, std::vector<float2>& out) {
 
 static int plan_upload(bpmh_plan p);
 
+// plans alive (guarded by g_loop_mu); the last one frees the buffers below
+static std::mutex g_loop_mu;
+static int g_plans = 0;
+static void loop_bufs_free();
+
 extern "C" int bpmh_plan_create(int nx, int ny, bpmh_plan* out) {
   if (!out) return bpmh_set_error(BPMH_ERR_INVALID, "null plan pointer");
   *out = nullptr;
@@ -995,6 +613,7 @@ extern "C" int bpmh_plan_create(int nx, int ny, bpmh_plan* out) {
   p->graph_mode = 0;
   p->cap_stream = nullptr;
   p->graph_clock = 0;
+  p->loop_mode = 0;
   p->device = -1;
   for (int e = 0; e < 2; ++e) {
     p->tw_x[e] = p->tw_y[e] = nullptr;
@@ -1012,6 +631,10 @@ extern "C" int bpmh_plan_create(int nx, int ny, bpmh_plan* out) {
     }
   } else {
     (void)hipGetLastError();
+  }
+  {
+    std::lock_guard<std::mutex> lock(g_loop_mu);
+    ++g_plans;
   }
   *out = p;
   return BPMH_OK;
@@ -1058,6 +681,8 @@ extern "C" int bpmh_plan_destroy(bpmh_plan p) {
   (void)graph_release_all(p);
   if (p->cap_stream) (void)hipStreamDestroy(p->cap_stream);
   delete p;
+  std::lock_guard<std::mutex> lock(g_loop_mu);
+  if (--g_plans == 0) loop_bufs_free();
   return BPMH_OK;
 }
 
@@ -1403,6 +1028,150 @@ static StepScratch prop_scratch_carve(bpmh_plan plan, const PropCall& c, void* b
   return r;
 }
 
+// ----------------------------------------------------------------------------
+// one-launch z-loop (loop.hpp): when it runs, and its synchronisation state
+// ----------------------------------------------------------------------------
+// Synchronisation words of the calls in flight, per device: a call takes a
+// buffer whose last user ran on the same stream (stream order protects it) or
+// has completed, so calls on several streams and host threads never share
+// one.  At most kLoopBufs buffers (each 12 KiB per team and XCD); beyond that
+// a call's stream waits for the buffer used longest ago.  They are freed with
+// the last plan.
+constexpr int kLoopBufs = 16;
+struct LoopBuf {
+  unsigned* ptr = nullptr;
+  size_t words = 0;
+  hipEvent_t last = nullptr;
+  hipStream_t stream = nullptr;
+  unsigned long long used = 0;  // 0: never
+};
+static LoopBuf g_loop_buf[64][kLoopBufs];
+static unsigned long long g_loop_clock = 0;
+
+// Called with g_loop_mu held; -1 and an error when none can be had.
+static int loop_buf_take(int dev, size_t words, hipStream_t s) {
+  LoopBuf* b = g_loop_buf[dev];
+  int pick = -1;
+  for (int i = 0; i < kLoopBufs && pick < 0; ++i)
+    if (b[i].used && b[i].stream == s && b[i].words >= words) pick = i;
+  for (int i = 0; i < kLoopBufs && pick < 0; ++i)
+    if (!b[i].used || (b[i].words >= words && hipEventQuery(b[i].last) == hipSuccess)) pick = i;
+  if (pick < 0) {
+    pick = 0;
+    for (int i = 1; i < kLoopBufs; ++i)
+      if (b[i].used < b[pick].used) pick = i;
+  }
+  LoopBuf& p = b[pick];
+  // (also on the same handle: another stream may have got a destroyed one's)
+  if (p.used && hipEventQuery(p.last) != hipSuccess && hipStreamWaitEvent(s, p.last, 0) != hipSuccess)
+    pick = -1;
+  (void)hipGetLastError();  // hipEventQuery's "not ready"
+  if (pick < 0) return -1;
+  if (p.words < words) {
+    if (p.used) (void)hipEventSynchronize(p.last);
+    if (p.ptr) (void)hipFree(p.ptr);
+    p.ptr = nullptr;
+    p.words = 0;
+    if (hipMalloc(&p.ptr, words * sizeof(unsigned)) != hipSuccess) {
+      p.ptr = nullptr;
+      (void)hipGetLastError();
+      return -1;
+    }
+    p.words = words;
+  }
+  if (!p.last && hipEventCreateWithFlags(&p.last, hipEventDisableTiming) != hipSuccess) return -1;
+  return pick;
+}
+
+static void loop_bufs_free() {
+  for (auto& dev : g_loop_buf)
+    for (LoopBuf& b : dev) {
+      if (b.used) (void)hipEventSynchronize(b.last);
+      if (b.ptr) (void)hipFree(b.ptr);
+      if (b.last) (void)hipEventDestroy(b.last);
+      b = LoopBuf();
+    }
+}
+
+__global__ void k_fill_zero(float* __restrict__ p, size_t n) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = 0.f;
+}
+
+// Whether a call of this grid, batch and schedule (er, ec points per thread of
+// rows and columns) runs as one launch.  By size: everywhere from 64^2 to
+// 512 x 256 (1.3 to 2.6 times faster, loop.hpp), except batches beyond 16 with
+// 1024-thread groups (512 x 256 at 4.4, batch 50: 83 against 70 us per step);
+// at 512^2, 32 CUs are too few for a field alone (batch 1: 14.0 against 12.5)
+// and only 8.8 fits two groups a CU (batch 2: 14.3 against 15.7; 16: 27.8
+// against 48; at 4.8 and batch 17 52.7 against 49.5).
+static bool loop_wanted(bpmh_plan plan, int batch, int nz, int er, int ec) {
+  const int nx = plan->nx, ny = plan->ny;
+  if (plan->loop_mode == 1 || nz < 2 || nx < 64 || ny < 64 || nx > 512 || ny > 512) return false;
+  if (!((er == 4 && ec == 4) || (er == 4 && ec == 8) || (er == 8 && ec == 8))) return false;  // not built
+  // fields of the records: 20 bits each for field, plane and sequence
+  if (nz >= (1 << 20) || (long long)batch * (nz / kLoopStepsPart + 2) >= (1 << 20)) return false;
+  if (plan->loop_mode >= 2) return true;
+  if (nx * ny == 512 * 512) return er == 8 && batch >= 2;
+  if (loop_points(nx, ny) == 4096 && ec == 4) return batch <= 16;
+  return true;
+}
+
+// Enqueue the z-loop of a call as one launch.  Returns 1 when done, 0 when
+// this call runs as launches per pass (size, schedule, or a stream that is
+// being captured: the synchronisation buffer must not be replayed), or an
+// error.
+static int loop_run(bpmh_plan plan, int mode, int batch, int nz, const LoopCall& call0, hipStream_t s) {
+  const int nx = plan->nx, ny = plan->ny;
+  const int er = row_e_of(nx, plan->row_v / kRowShapes), ec = col_e_of(ny, plan->col_v / kColShapes);
+  if (!loop_wanted(plan, batch, nz, er, ec)) return 0;
+  loop_launch_fn launch = nx == 64    ? bpmh_loop_nx64
+                          : nx == 128 ? bpmh_loop_nx128
+                          : nx == 256 ? bpmh_loop_nx256
+                                      : bpmh_loop_nx512;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  int dev = -1;
+  HIP_TRY(hipGetDevice(&dev));
+  if (dev != plan->device || dev < 0 || dev >= 64) return 0;
+  LoopCall call = call0;
+  const int slots = loop_slots(nx, ny);
+  // teams per XCD: one per field up to what the XCD's 32 CUs hold
+  int teams = (batch + 7) / 8;
+  const int most = 256 / slots < 1 ? 1 : 256 / slots;
+  if (teams > most) teams = most;
+  call.la.batch = batch;
+  call.la.teams = teams;
+  const size_t words = loop_words(teams);
+  std::lock_guard<std::mutex> lock(g_loop_mu);
+  const int i = loop_buf_take(dev, words, s);
+  if (i < 0) return 0;
+  LoopBuf& b = g_loop_buf[dev][i];
+  call.la.sync = b.ptr;
+  hipLaunchKernelGGL(k_fill_zero, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, s, (float*)b.ptr,
+                     words);
+  const int groups = 8 * teams * slots;
+  const bool ok = launch(ny, er, ec, mode, call, plan->loop_mode == 3 ? groups / 4 : groups, s);
+  const hipError_t le = hipGetLastError();
+  const hipError_t re = hipEventRecord(b.last, s);
+  b.stream = s;
+  b.used = ++g_loop_clock;
+  if (!ok) return 0;
+  if (le != hipSuccess || re != hipSuccess)
+    return bpmh_set_error(BPMH_ERR_HIP, hipGetErrorString(le != hipSuccess ? le : re));
+  return 1;
+}
+
+extern "C" int bpmh_plan_set_loop(bpmh_plan p, int mode) {
+  if (!p) return bpmh_set_error(BPMH_ERR_INVALID, "null plan");
+  if (mode < 0 || mode > 3) return bpmh_set_error(BPMH_ERR_INVALID, "loop mode is 0 to 3");
+  p->loop_mode = mode;
+  return BPMH_OK;
+}
+
 // Enqueue (or capture and replay) the whole z-loop of one call on stream s.
 // may_allocate false: plain launches only (no graph capture or timing
 // events, which create runtime objects).
@@ -1462,6 +1231,21 @@ static int prop_run(bpmh_plan plan, const PropCall& c, const StepScratch& sc, hi
   ca.spart = sc.spart;
 
   const bool timing = may_allocate && plan->timing;
+  if (may_allocate && !timing) {
+    LoopCall call;
+    memset(&call, 0, sizeof call);
+    call.ra = ra;
+    call.ca = ca;
+    const int rc = loop_run(plan, c.mean_mode, batch, nz, call, s);
+    if (rc < 0) return rc;
+    if (rc == 1) {
+      if (c.out_scat)
+        hipLaunchKernelGGL(k_scatter_final, dim3((nz + 63) / 64, batch), dim3(64), 0, s, sc.spart,
+                           c.out_scat, nz, nx);
+      HIP_TRY(hipGetLastError());
+      return BPMH_OK;
+    }
+  }
   if (timing) {
     const int rc = timing_reserve(plan, (size_t)nz * 3 + 1);
     if (rc) return rc;
@@ -1776,6 +1560,50 @@ extern "C" int bpmh_propagate(bpmh_plan plan, int batch, int nz, float* plane, c
 // ----------------------------------------------------------------------------
 // ragged batch: groups of fields with their own dn volumes and depths
 // ----------------------------------------------------------------------------
+// The launches per pass of a ragged batch: group g of items[g] fields, depth
+// nzs[g]; events as in bpmh_propagate_groups.
+static int groups_launches(row_fn row, col_fn col, RowArgs ra, ColArgs ca, int dn_kind, int n_groups,
+                           const int* items, const int* nzs, int total, void** group_done,
+                           hipStream_t s) {
+  // items still propagating at plane z (and, for the forward transform, past
+  // it): a prefix, the groups being in order of non-increasing depth
+  auto items_deeper = [&](int z) {
+    int c = 0;
+    for (int g = 0; g < n_groups; ++g)
+      if (nzs[g] > z) c += items[g];
+    return c;
+  };
+  auto mark_done = [&](int z) -> int {  // groups whose last plane is z
+    if (!group_done) return BPMH_OK;
+    for (int g = 0; g < n_groups; ++g)
+      if (nzs[g] - 1 == z && group_done[g]) HIP_TRY(hipEventRecord((hipEvent_t)group_done[g], s));
+    return BPMH_OK;
+  };
+  ra.z = 0;
+  ra.acc_init = 1;
+  ra.inverse = 0;
+  ra.screen = 0;
+  ra.fwd_items = items_deeper(1);
+  row(ra, total, s);
+  int rc = mark_done(0);
+  if (rc) return rc;
+  ra.acc_init = 0;
+  ra.inverse = 1;
+  ra.screen = dn_kind != BPMH_DN_NONE;
+  for (int z = 1; z < nzs[0]; ++z) {
+    const int active = items_deeper(z);
+    ca.z = z;
+    col(ca, active, s);
+    ra.z = z;
+    ra.fwd_items = items_deeper(z + 1);
+    row(ra, active, s);
+    rc = mark_done(z);
+    if (rc) return rc;
+  }
+  HIP_TRY(hipGetLastError());
+  return BPMH_OK;
+}
+
 extern "C" int bpmh_propagate_groups(bpmh_plan plan, int n_groups, const int* items,
                                      const int* nzs, float* plane_, const void* dn, int dn_kind,
                                      long long dn_group_stride, long long dn_numel,
@@ -1844,43 +1672,42 @@ extern "C" int bpmh_propagate_groups(bpmh_plan plan, int n_groups, const int* it
   ca.hmode = 0;
   ca.H = H;
 
-  // items still propagating at plane z (and, for the forward transform, past
-  // it): a prefix, the groups being in order of non-increasing depth
-  auto items_deeper = [&](int z) {
-    int c = 0;
-    for (int g = 0; g < n_groups; ++g)
-      if (nzs[g] > z) c += items[g];
-    return c;
-  };
-  auto mark_done = [&](int z) -> int {  // groups whose last plane is z
-    if (!group_done) return BPMH_OK;
-    for (int g = 0; g < n_groups; ++g)
-      if (nzs[g] - 1 == z && group_done[g]) HIP_TRY(hipEventRecord((hipEvent_t)group_done[g], s));
-    return BPMH_OK;
-  };
-  ra.z = 0;
-  ra.acc_init = 1;
-  ra.inverse = 0;
-  ra.screen = 0;
-  ra.fwd_items = items_deeper(1);
-  row(ra, total, s);
-  rc = mark_done(0);
-  if (rc) return rc;
-  ra.acc_init = 0;
-  ra.inverse = 1;
-  ra.screen = dn_kind != BPMH_DN_NONE;
-  for (int z = 1; z < nzs[0]; ++z) {
-    const int active = items_deeper(z);
-    ca.z = z;
-    col(ca, active, s);
-    ra.z = z;
-    ra.fwd_items = items_deeper(z + 1);
-    row(ra, active, s);
-    rc = mark_done(z);
-    if (rc) return rc;
+  // One launch.  Groups that report their completion separately run one after
+  // another, the shallowest first, so that each event fires when its group is
+  // done.
+  LoopCall call;
+  memset(&call, 0, sizeof call);
+  call.ra = ra;
+  call.ca = ca;
+  if (!group_done || n_groups == 1) {
+    for (int g = 0; g < n_groups; ++g) call.la.gnz[g] = nzs[g];
+    rc = loop_run(plan, BPMH_MEAN_IGNORE, total, nzs[0], call, s);
+    if (rc < 0) return rc;
+    if (rc == 1) {
+      if (group_done && group_done[0]) HIP_TRY(hipEventRecord((hipEvent_t)group_done[0], s));
+      return BPMH_OK;
+    }
+    return groups_launches(row, col, ra, ca, dn_kind, n_groups, items, nzs, total, group_done, s);
   }
-  HIP_TRY(hipGetLastError());
-  return BPMH_OK;
+  const size_t dn_size = dn_kind == BPMH_DN_F16 ? 2 : (dn_kind == BPMH_DN_C64 ? 8 : 4);
+  int g = n_groups;
+  for (int first = total; g > 0; --g) {
+    first -= items[g - 1];
+    call.ra.plane = call.ca.plane = plane + (size_t)first * n;
+    call.ra.acc = out_sum ? out_sum + (size_t)first * n : nullptr;
+    if (dn) call.ra.dn = (const char*)dn + (size_t)(g - 1) * dn_group_stride * dn_size;
+    call.ra.ngroups = 0;
+    call.ra.dn_bstride = 0;
+    call.ra.nz = call.ca.nz = nzs[g - 1];
+    rc = loop_run(plan, BPMH_MEAN_IGNORE, items[g - 1], nzs[g - 1], call, s);
+    if (rc < 0) return rc;
+    if (rc == 0) break;
+    if (group_done[g - 1]) HIP_TRY(hipEventRecord((hipEvent_t)group_done[g - 1], s));
+    total = first;
+  }
+  if (g == 0) return BPMH_OK;
+  // the groups left (all of them, unless a synchronisation buffer ran out)
+  return groups_launches(row, col, ra, ca, dn_kind, g, items, nzs, total, group_done, s);
 }
 
 // ----------------------------------------------------------------------------
@@ -2094,11 +1921,6 @@ __global__ void __launch_bounds__(256) k_row_sums(const float* __restrict__ g,
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
   if (lane == 0) out[r] = sum;
-}
-
-__global__ void k_fill_zero(float* __restrict__ p, size_t n) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0.f;
 }
 
 // Workspace of bpmh_mean_segment, in floats (each part 256-byte aligned).

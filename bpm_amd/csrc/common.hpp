@@ -95,26 +95,29 @@ BPMH_DEV float2 sincos_f32_via_f64(float ph) {
   return make_float2((q == 1 || q == 2) ? -a : a, (q & 2) ? -b : b);
 }
 
-// sin and cos of a float32 angle.  For |x| <= pi/4 (every phase screen of a
-// physical index contrast: |k0 dz dn| is far below that) the Taylor series of
-// sin to x^9 and cos to x^10, in Horner form with FMA; the first omitted terms
-// are below 2.5e-9 relative, so the result is within about 1 ulp.  Larger
-// arguments go to the range-reduced library sincosf.
+// sin and cos of |x| <= pi/4 by the Taylor series of sin to x^9 and cos to
+// x^10, in Horner form with FMA; the first omitted terms are below 2.5e-9
+// relative, so the result is within about 1 ulp.
+constexpr float kSincosNear = 0.78539816f;
+BPMH_DEV void sincos_near(float x, float* s, float* c) {
+  const float x2 = x * x;
+  float ps = fmaf(x2, 2.75573192e-6f, -1.98412698e-4f);  // 1/9!, -1/7!
+  ps = fmaf(x2, ps, 8.33333333e-3f);                      // 1/5!
+  ps = fmaf(x2, ps, -1.66666667e-1f);                     // -1/3!
+  *s = fmaf(x * x2, ps, x);
+  float pc = fmaf(x2, -2.75573192e-7f, 2.48015873e-5f);   // -1/10!, 1/8!
+  pc = fmaf(x2, pc, -1.38888889e-3f);                     // -1/6!
+  pc = fmaf(x2, pc, 4.16666667e-2f);                      // 1/4!
+  pc = fmaf(x2, pc, -0.5f);
+  *c = fmaf(x2, pc, 1.f);
+}
+
+// sin and cos of a float32 angle: the series up to pi/4 (every phase screen
+// of a physical index contrast: |k0 dz dn| is far below that), the
+// range-reduced library sincosf beyond.
 BPMH_DEV void sincos_fast(float x, float* s, float* c) {
-  if (fabsf(x) <= 0.78539816f) {
-    const float x2 = x * x;
-    float ps = fmaf(x2, 2.75573192e-6f, -1.98412698e-4f);  // 1/9!, -1/7!
-    ps = fmaf(x2, ps, 8.33333333e-3f);                      // 1/5!
-    ps = fmaf(x2, ps, -1.66666667e-1f);                     // -1/3!
-    *s = fmaf(x * x2, ps, x);
-    float pc = fmaf(x2, -2.75573192e-7f, 2.48015873e-5f);   // -1/10!, 1/8!
-    pc = fmaf(x2, pc, -1.38888889e-3f);                     // -1/6!
-    pc = fmaf(x2, pc, 4.16666667e-2f);                      // 1/4!
-    pc = fmaf(x2, pc, -0.5f);
-    *c = fmaf(x2, pc, 1.f);
-  } else {
-    sincosf(x, s, c);
-  }
+  if (fabsf(x) <= kSincosNear) sincos_near(x, s, c);
+  else sincosf(x, s, c);
 }
 
 // Streaming (nontemporal) global accesses.  Used where measurement favours

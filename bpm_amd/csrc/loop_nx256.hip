@@ -1,0 +1,6 @@
+// The one-launch z-loop (loop.hpp) for rows of 256 points.
+#include "loop.hpp"
+
+bool bpmh_loop_nx256(int ny, int er, int ec, int mode, const LoopCall& c, int groups, hipStream_t s) {
+  return loop_launch_nx<256>(ny, er, ec, mode, c, groups, s);
+}

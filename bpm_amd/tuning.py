@@ -5,7 +5,10 @@ For a grid (Nx, Ny) and batch size it times every (row, column) variant of
 accesses, and for each pass both radix schedules (4 or 8 elements per
 thread, e.g. a 1024-point line as 4.4.4.4.4 or 2.8.8.8) -- on the device
 (HIP events on the current stream around a short propagation) and keeps the
-fastest.  Results are cached in
+fastest.  Grids that run their z-loop as one launch (bpmh_plan_set_loop) have
+one time per schedule there; the schedule with the fastest loop is kept, with
+the launch shapes that are its fastest as launches per pass (which timed,
+captured and adjoint passes still use).  Results are cached in
 ``tuning_cache.json`` next to the library, keyed by "gfx:NxxNy:batch";
 ``get_plan`` applies a cached choice automatically.
 """
@@ -35,17 +38,24 @@ def load_cache():
     return _cache
 
 
+_index = (None, {})  # (cache it was made from, {(nx, ny): [(batch, best), ...]})
+
+
 def lookup(nx, ny, batch=1):
     """Cached (row_variant, col_variant) for this grid and batch, else for
     the nearest cached batch of the same grid, else None."""
+    global _index
     c = load_cache()
-    k = _key(nx, ny, batch)
-    if k in c:
-        return tuple(c[k]["best"])
-    same = [(abs(int(v.split(":")[2]) - batch), v) for v in c if v.split(":")[1] == "%dx%d" % (nx, ny)]
-    if same:
-        return tuple(c[min(same)[1]]["best"])
-    return None
+    if _index[0] is not c or sum(len(v) for v in _index[1].values()) != len(c):
+        grids = {}
+        for k, v in c.items():
+            _, grid, b = k.split(":")
+            grids.setdefault(tuple(int(n) for n in grid.split("x")), []).append((int(b), tuple(v["best"])))
+        _index = (c, grids)
+    same = _index[1].get((nx, ny))
+    if not same:
+        return None
+    return min(same, key=lambda e: (abs(e[0] - batch), e[0]))[1]
 
 
 ROW_VARIANTS, COL_VARIANTS = 6, 10  # V + 3*s, V + 5*s (s: radix schedule)
@@ -61,7 +71,9 @@ def shape_of(plan):
 
 def autotune(nx, ny, batch=1, nz=65, reps=3, units=(.1, .1, .1), lam=.5, n0=1.33, save=None):
     """Time all 6x10 (row, column) variants for one grid/batch (variants that
-    map to an identical kernel pair are timed once); returns (best, table)."""
+    map to an identical kernel pair are timed once) and each schedule as the
+    plan runs it; returns (best, table), the table of the kept schedule's
+    launch shapes where the grid is one of the one-launch sizes."""
     from . import bpm3d as B
     t = _lib.torch()
     plan = B.get_plan(nx, ny, None)
@@ -71,7 +83,25 @@ def autotune(nx, ny, batch=1, nz=65, reps=3, units=(.1, .1, .1), lam=.5, n0=1.33
     H = B.propagator_table(nx, ny, units, lam, n0, _lib.H_F64)
     acc = t.empty((batch, ny, nx), dtype=t.float32, device=_lib.device())
     plane = t.empty_like(u0)
+
+    def run():
+        plane.copy_(u0)
+        B.propagate_fields(plane, nz, units, lam, n0, dn=dn, dn_kind=_lib.DN_F32,
+                           mean_mode="ignore", H=H, out_sum=acc, tuned=False)
+
+    def time_ms():
+        run()
+        t.cuda.synchronize()
+        e0, e1 = t.cuda.Event(enable_timing=True), t.cuda.Event(enable_timing=True)
+        e0.record()
+        for _ in range(reps):
+            run()
+        e1.record()
+        t.cuda.synchronize()
+        return e0.elapsed_time(e1) / reps
+
     table = {}
+    _lib.call("bpmh_plan_set_loop", plan, 1)
     for rv in range(ROW_VARIANTS):
         for cv in range(COL_VARIANTS):
             _lib.call("bpmh_plan_set_variant", plan, rv, cv)
@@ -81,26 +111,26 @@ def autotune(nx, ny, batch=1, nz=65, reps=3, units=(.1, .1, .1), lam=.5, n0=1.33
                 key.append(cv % 5)  # paired / split columns: kernels of their own
             if key in [v["shape"] for v in table.values()]:
                 continue  # clamped to an identical launch shape
-            def run():
-                plane.copy_(u0)
-                B.propagate_fields(plane, nz, units, lam, n0, dn=dn, dn_kind=_lib.DN_F32,
-                                   mean_mode="ignore", H=H, out_sum=acc, tuned=False)
-            run()
-            t.cuda.synchronize()
-            e0, e1 = t.cuda.Event(enable_timing=True), t.cuda.Event(enable_timing=True)
-            e0.record()
-            for _ in range(reps):
-                run()
-            e1.record()
-            t.cuda.synchronize()
-            ms = e0.elapsed_time(e1) / reps
+            ms = time_ms()
             table["%d,%d" % (rv, cv)] = {"ms": ms, "shape": key,
                                          "us_per_step": ms * 1e3 / (nz - 1)}
+    _lib.call("bpmh_plan_set_loop", plan, 0)
+    # the time of each schedule as it runs, at its fastest launch shapes
+    runs = {}
+    for sched in {tuple(v["shape"][2:4]) for v in table.values()}:
+        k = min((k for k in table if tuple(table[k]["shape"][2:4]) == sched), key=lambda k: table[k]["ms"])
+        _lib.call("bpmh_plan_set_variant", plan, *(int(x) for x in k.split(",")))
+        runs[sched] = (time_ms(), k)
+    sched = min(runs, key=lambda q: runs[q][0])
+    best = runs[sched][1]
+    loop_us = {"%d.%d" % q: r[0] * 1e3 / (nz - 1) for q, r in runs.items()}
+    if nx <= 512 and ny <= 512 and min(nx, ny) >= 64:
+        table = {k: v for k, v in table.items() if tuple(v["shape"][2:4]) == sched}
     best = min(table, key=lambda k: table[k]["ms"])
     bv = tuple(int(x) for x in best.split(","))
     _lib.call("bpmh_plan_set_variant", plan, *bv)
     c = load_cache()
-    c[_key(nx, ny, batch)] = {"best": list(bv), "table": table}
+    c[_key(nx, ny, batch)] = {"best": list(bv), "table": table, "us_per_step": loop_us}
     if save:
         with open(save, "w") as f:
             json.dump(c, f, indent=1, sort_keys=True)

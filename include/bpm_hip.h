@@ -78,8 +78,19 @@ int bpmh_plan_kernel_times(bpmh_plan plan, float* ms, int* counts);
  * destroyed (on eviction, on bpmh_plan_set_graph(plan, 0) and at
  * bpmh_plan_destroy) only after its latest replay has completed.  Replaces
  * the per-kernel Python->pyopencl enqueue of the reference loop
- * (bpm/bpm/bpm_3d.py:283-382).  Ignored while timing is on. */
+ * (bpm/bpm/bpm_3d.py:283-382).  Ignored while timing is on, and for calls
+ * that run as one launch (bpmh_plan_set_loop). */
 int bpmh_plan_set_graph(bpmh_plan plan, int enable);
+
+/* How bpmh_propagate, bpmh_propagate_groups and the recorded forward of
+ * bpmh_mean_segment run grids of 64 to 512 points a side: 0 (default) one
+ * launch for the whole z-loop where it measured faster, by grid and batch;
+ * 1 always one launch per pass; 2 one launch wherever it is built; 3 as 2
+ * with a quarter of its work-groups (what a busy GPU may leave it at first;
+ * for tests).  The results are the same bits.  Streams that are being captured, timed plans
+ * and bpmh_propagate_noalloc always use one launch per pass.  No reference
+ * counterpart. */
+int bpmh_plan_set_loop(bpmh_plan plan, int mode);
 
 /* Launch-shape and radix-schedule variants of the row and column passes,
  * chosen per grid size and batch by the autotuner (bpm_amd/tuning.py).
