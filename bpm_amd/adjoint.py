@@ -29,7 +29,9 @@ in the field gradient and the gradient of slice 0.  With
 dL/ddn0 / N is added to every voxel of that plane.  Real dn only.
 
 Memory: checkpoints B*ceil(nz/K) planes + one segment of B*(K+1) planes
-(weighted: about 2*B*(K+2) planes of recorded forward state).
+(weighted: about 2*B*(K+2) planes of recorded forward state); where a segment's
+adjoint runs as one launch (grids of 64 to 512 points a side) the screen
+gradients of every step, B*K real planes, instead of B.
 """
 import ctypes
 
@@ -75,19 +77,22 @@ def _make_fn():
             Bn = grad_out.shape[0]
             g = grad_out.to(dtype=t.complex64).contiguous().clone()
             grad_dn = t.zeros_like(dnc)
-            gitem = t.empty((Bn, ny, nx), dtype=dnc.dtype, device=dnc.device)
             k0dz = float(np.float32(2. * np.pi / lam * units[2]))
-            plan = B.get_plan(nx, ny)
+            plan = B.get_plan(nx, ny, Bn)
+            need = ctypes.c_longlong()
+            _lib.call("bpmh_adjoint_segment_work", plan, int(Bn), 0, max(z1 - z0 for z0, z1 in segs)
+                      if segs else 0, int(kind), ctypes.byref(need))
+            work = t.empty(int(need.value), dtype=t.float32, device=dnc.device)
             for (z0, z1), ck in zip(reversed(segs), reversed(ckpts)):
                 useg = t.empty((Bn, z1 - z0 + 1, ny, nx), dtype=t.complex64, device=dnc.device)
                 p = ck.clone()
                 B.propagate_fields(p, z1 - z0 + 1, units, lam, n0, dn=dnc[z0:],
                                    dn_kind=kind, mean_mode="ignore", H=H,
                                    absorbing_width=absorb, out_field=useg)
-                _lib.call("bpmh_adjoint_segment", plan, int(Bn), int(z0), int(z1), _lib.ptr(g),
+                _lib.call("bpmh_adjoint_segment_ws", plan, int(Bn), int(z0), int(z1), _lib.ptr(g),
                           _lib.ptr(useg), int(useg.numel()), _lib.ptr(dnc), int(kind),
                           int(dnc.numel()), _lib.ptr(H), k0dz, int(absorb), _lib.ptr(grad_dn),
-                          _lib.ptr(gitem), _lib.stream_handle())
+                          _lib.ptr(work), int(work.numel()), _lib.stream_handle())
             return grad_dn, g, None, None, None, None, None
 
     return _Fn
@@ -103,7 +108,7 @@ def _mean_args(units, lam, n0):
 def _mean_call(mode, plane, z0, z1, dnc, means, consts, absorb, g, grad_dn, work):
     n0, k0, dx, dy, dz, unit_k = consts
     n_eff, dn0 = means if means is not None else (None, None)
-    _lib.call("bpmh_mean_segment", B.get_plan(dnc.shape[2], dnc.shape[1]), int(mode),
+    _lib.call("bpmh_mean_segment", B.get_plan(dnc.shape[2], dnc.shape[1], plane.shape[0]), int(mode),
               int(plane.shape[0]), int(z0), int(z1), _lib.ptr(plane), _lib.ptr(dnc),
               int(dnc.numel()), _lib.ptr(n_eff), _lib.ptr(dn0), n0, k0, dx, dy, dz, unit_k,
               int(absorb), _lib.ptr(g) if g is not None else None,
@@ -114,7 +119,7 @@ def _mean_call(mode, plane, z0, z1, dnc, means, consts, absorb, g, grad_dn, work
 def _work(nx, ny, batch, z0, z1, adjoint):
     t = _lib.torch()
     n = ctypes.c_longlong()
-    _lib.call("bpmh_mean_segment_work", B.get_plan(nx, ny), int(batch), int(z0), int(z1),
+    _lib.call("bpmh_mean_segment_work", B.get_plan(nx, ny, batch), int(batch), int(z0), int(z1),
               int(adjoint), ctypes.byref(n))
     return t.empty(int(n.value), dtype=t.float32, device=_lib.device())
 

@@ -16,6 +16,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libbpmhip.so")
 SOURCES = ["bpm_kernels.hip", "loop_nx64.hip", "loop_nx128.hip", "loop_nx256.hip", "loop_nx512.hip",
+           "loop_adj_nx64.hip", "loop_adj_nx128.hip", "loop_adj_nx256.hip", "loop_adj_nx512.hip",
            "debye.hip", "spheres.hip"]
 ARCH = os.environ.get("BPMH_OFFLOAD_ARCH", "gfx950")
 
@@ -40,7 +41,7 @@ def _compile(src):
 def build(verbose=True):
     """Compile every source and link libbpmhip.so; returns the library path."""
     os.makedirs(BUILD, exist_ok=True)
-    with ThreadPoolExecutor(max_workers=len(SOURCES)) as ex:
+    with ThreadPoolExecutor(max_workers=min(len(SOURCES), os.cpu_count() or 1, 16)) as ex:
         objs = list(ex.map(_compile, SOURCES))
     tmp = LIB + ".tmp"
     cmd = [HIPCC, "--offload-arch=" + ARCH, "-shared", "-fPIC", "-o", tmp] + objs

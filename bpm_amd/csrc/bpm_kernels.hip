@@ -14,7 +14,7 @@
 // default mean_mode "weighted" of bpm_3d needs the k-space reduction of
 // bpm_3d.py:302-303 before H, so its column pass is split in two (A: FFT_y
 // and per-column partial sums; B: H(n0+dn0) and IFFT_y).
-#include "loop.hpp"
+#include "loop_adj.hpp"
 
 #include <cmath>
 #include <cstdint>
@@ -249,7 +249,7 @@ k_col(ColArgs a) {
     const float2 sums = group_sum_pair(a.s1part + (size_t)b * NY, NY, a.s2part + (size_t)b * a.nx,
                                        a.nx, cg_slot);
     n_pts = (float)a.nx * (float)NY;
-    cgrad = -sums.x + a.dz * n_adj * a.k0 * a.k0 / n_pts * sums.y;
+    cgrad = adjoint_cgrad(sums.x, sums.y, a.dz, n_adj, a.k0, n_pts);
     if (a.simple) {
       if (bx == 0 && threadIdx.x == 0) a.cg_out[b] = cgrad;
     } else {
@@ -288,44 +288,11 @@ k_col(ColArgs a) {
       // dH/ddn0 = H * (-i dz (n0+dn0) k0^2 / beta): collect Im(conj(X) H U)/beta
       const float an = n_term_f32(n_adj, a.k0);
       const float kx2 = kcomp2_f32(x, a.nx, a.dx);
-      // H and beta for half the rows, the mirrored rows (same values bit for
-      // bit) from the partner thread through the line, as in the H passes
       float2 h[E];
       float bt[E];
-#pragma unroll
-      for (int m = 0; m < E / 2; ++m)
-        h[m] = prop_f32_beta(kx2, kcomp2_f32(t + m * T, NY, a.dy), an, a.dz, &bt[m]);
-      if (t == 0)
-        h[E / 2] = prop_f32_beta(kx2, kcomp2_f32(NY / 2, NY, a.dy), an, a.dz, &bt[E / 2]);
-      __syncthreads();  // earlier users of the line are done with it
-#pragma unroll
-      for (int m = 0; m < E / 2; ++m) {
-        line[m * T + t] = h[m];
-        line[NY / 2 + m * T + t] = make_float2(bt[m], 0.f);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int m = E / 2; m < E; ++m) {
-        if (t == 0) {
-          if (m > E / 2) {
-            h[m] = h[E - m];
-            bt[m] = bt[E - m];
-          }
-        } else {
-          h[m] = line[(E - 1 - m) * T + T - t];
-          bt[m] = line[NY / 2 + (E - 1 - m) * T + T - t].x;
-        }
-      }
-      float acc = 0.f;  // (column_sum2 waits for every reader of the line)
-#pragma unroll
-      for (int m = 0; m < E; ++m) {
-        if (bt[m] > 0.f) {
-          const float2 hu = c_mul(h[m], uv[q][m]);
-          acc += (v[q][m].x * hu.y - v[q][m].y * hu.x) / bt[m];
-        }
-      }
-      const float2 tot = column_sum2<T>(make_float2(acc, 0.f), line, t);
-      if (t == 0) a.s2part[(size_t)b * a.nx + x] = tot.x;
+      col_hb_fly<NY, E>(kx2, an, a.dy, a.dz, t, line, h, bt);
+      const float tot = col_beta_sum<NY, E>(v[q], h, uv[q], bt, t, line);
+      if (t == 0) a.s2part[(size_t)b * a.nx + x] = tot;
     } else {
       float an = 0.f, kx2 = 0.f;
       if (a.hmode != 0) {
@@ -351,21 +318,11 @@ k_col(ColArgs a) {
         }
       }
       if (PHASE == 4 && !a.simple) {
-        // dn0 = sum|U| d / sum|U| depends on U through |U|:
-        // G_U += dL/ddn0 (d - dn0) / W * U/|U| (times N: X is N G_V), and
-        // dL/dd += dL/ddn0 |U| / W
         float* gd = a.gd_item + (size_t)b * NY * a.nx + x;
 #pragma unroll
-        for (int m = 0; m < E; ++m) {
-          const int ky = t + m * T;
-          const float au = hypotf(uv[q][m].x, uv[q][m].y);
-          if (au > 0.f) {
-            const float coef = n_pts * cgrad * (dv[q][m] - dn0w) * inv_w / au;
-            v[q][m].x += coef * uv[q][m].x;
-            v[q][m].y += coef * uv[q][m].y;
-          }
-          gd[(size_t)ky * a.nx] += cgrad * au * inv_w;
-        }
+        for (int m = 0; m < E; ++m)
+          gd[(size_t)(t + m * T) * a.nx] +=
+              adjoint_weight_term(v[q][m], uv[q][m], dv[q][m], dn0w, cgrad, inv_w, n_pts);
       }
       if (a.sw) col_scatter<NY, E>(a, a.z, b, x, t, line, v[q]);
     }
@@ -1098,6 +1055,10 @@ __global__ void k_fill_zero(float* __restrict__ p, size_t n) {
   if (i < n) p[i] = 0.f;
 }
 
+static bool loop_size(bpmh_plan plan) {
+  return plan->nx >= 64 && plan->ny >= 64 && plan->nx <= 512 && plan->ny <= 512;
+}
+
 // Whether a call of this grid, batch and schedule (er, ec points per thread of
 // rows and columns) runs as one launch.  By size: everywhere from 64^2 to
 // 512 x 256 (1.3 to 2.6 times faster, loop.hpp), except batches beyond 16 with
@@ -1107,7 +1068,7 @@ __global__ void k_fill_zero(float* __restrict__ p, size_t n) {
 // against 48; at 4.8 and batch 17 52.7 against 49.5).
 static bool loop_wanted(bpmh_plan plan, int batch, int nz, int er, int ec) {
   const int nx = plan->nx, ny = plan->ny;
-  if (plan->loop_mode == 1 || nz < 2 || nx < 64 || ny < 64 || nx > 512 || ny > 512) return false;
+  if (plan->loop_mode == 1 || nz < 2 || !loop_size(plan)) return false;
   if (!((er == 4 && ec == 4) || (er == 4 && ec == 8) || (er == 8 && ec == 8))) return false;  // not built
   // fields of the records: 20 bits each for field, plane and sequence
   if (nz >= (1 << 20) || (long long)batch * (nz / kLoopStepsPart + 2) >= (1 << 20)) return false;
@@ -1117,18 +1078,36 @@ static bool loop_wanted(bpmh_plan plan, int batch, int nz, int er, int ec) {
   return true;
 }
 
-// Enqueue the z-loop of a call as one launch.  Returns 1 when done, 0 when
-// this call runs as launches per pass (size, schedule, or a stream that is
-// being captured: the synchronisation buffer must not be replayed), or an
-// error.
-static int loop_run(bpmh_plan plan, int mode, int batch, int nz, const LoopCall& call0, hipStream_t s) {
+// The same for the adjoint of a segment of nz planes.  Not built for rows of
+// more than one wavefront; the reduction's grid has a block row per plane.
+// Without a mean correction a step is short beside the forward planes it reads
+// and the screen gradients it writes, so from 512 x 256 on only while the
+// teams take the batch in one round (512^2 at 8.8, batch 8: 34 against 39 us
+// per step, 16: 68 against 59; 512 x 256, batch 1: 16.3 against 15.7, 16: 33
+// against 38, 50: 112 against 88; 256^2, batch 50: 37 against 55).  With one
+// it is 1.1 to 2.1 times faster throughout (512^2 at 8.8, batch 8: 81 against
+// 120, 50: 544 against 622).
+static bool loop_adj_wanted(bpmh_plan plan, int mode, int batch, int nz, int er, int ec) {
+  const long long pts = (long long)plan->nx * plan->ny;
+  if (!loop_wanted(plan, batch, nz, er, ec) || plan->nx / er > 64 || nz > 65536) return false;
+  if (plan->loop_mode >= 2 || mode != BPMH_MEAN_IGNORE || pts < 512 * 256) return true;
+  return batch >= 2 && batch * pts <= 8LL * 512 * 512;
+}
+
+// Enqueue the z-loop of a call (adj: the adjoint of a segment of nz planes) as
+// one launch.  Returns 1 when done, 0 when this call runs as launches per pass
+// (size, schedule, or a stream that is being captured: the synchronisation
+// buffer must not be replayed), or an error.
+static int loop_run(bpmh_plan plan, int mode, int batch, int nz, const LoopCall& call0, hipStream_t s,
+                    bool adj = false) {
   const int nx = plan->nx, ny = plan->ny;
   const int er = row_e_of(nx, plan->row_v / kRowShapes), ec = col_e_of(ny, plan->col_v / kColShapes);
-  if (!loop_wanted(plan, batch, nz, er, ec)) return 0;
-  loop_launch_fn launch = nx == 64    ? bpmh_loop_nx64
-                          : nx == 128 ? bpmh_loop_nx128
-                          : nx == 256 ? bpmh_loop_nx256
-                                      : bpmh_loop_nx512;
+  if (!(adj ? loop_adj_wanted(plan, mode, batch, nz, er, ec) : loop_wanted(plan, batch, nz, er, ec)))
+    return 0;
+  loop_launch_fn launch = nx == 64    ? (adj ? bpmh_loop_adj_nx64 : bpmh_loop_nx64)
+                          : nx == 128 ? (adj ? bpmh_loop_adj_nx128 : bpmh_loop_nx128)
+                          : nx == 256 ? (adj ? bpmh_loop_adj_nx256 : bpmh_loop_nx256)
+                                      : (adj ? bpmh_loop_adj_nx512 : bpmh_loop_nx512);
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
     (void)hipGetLastError();
@@ -1809,22 +1788,35 @@ extern "C" int bpmh_propagate_noalloc(bpmh_plan plan, int batch, int nz, float* 
 // ----------------------------------------------------------------------------
 // adjoint (gradient of a loss on the last plane with respect to dn)
 // ----------------------------------------------------------------------------
-// grad[i] += sum_b gitem[b][i] in item order (deterministic); n counts floats
-// (one per voxel for real dn, two for complex dn)
-__global__ void k_grad_reduce(const float* __restrict__ gitem, float* __restrict__ grad,
-                              int batch, size_t n) {
+// Per plane p: grad[p][i] += sum_b gitem[p][b][i] in item order (deterministic),
+// then, with cg, (sum_b cg[p][b]) * inv_n: dL/ddn0 of a simple-mean step spread
+// over the plane that dn0 is the mean of.  n counts floats (one per voxel for
+// real dn, two for complex dn).
+__global__ void k_grad_reduce(const float* __restrict__ gitem, float* __restrict__ grad, int batch,
+                              size_t n, const float* __restrict__ cg, float inv_n) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  float s = grad[i];
-  for (int b = 0; b < batch; ++b) s += gitem[(size_t)b * n + i];
-  grad[i] = s;
+  const size_t p = blockIdx.y;
+  float s = grad[p * n + i];
+  for (int b = 0; b < batch; ++b) s += gitem[(p * batch + b) * n + i];
+  if (cg) {
+    float c = 0.f;
+    for (int b = 0; b < batch; ++b) c += cg[p * batch + b];
+    s += c * inv_n;
+  }
+  grad[p * n + i] = s;
 }
 
-extern "C" int bpmh_adjoint_segment(bpmh_plan plan, int batch, int z_lo, int z_hi, float* g_,
-                                    const float* u_seg_, long long u_seg_numel, const void* dn,
-                                    int dn_kind, long long dn_numel, const float* H_,
-                                    float unit_k, int absorb, float* grad_dn, float* gitem,
-                                    void* stream) {
+static void launch_grad_reduce(const float* gitem, float* grad, int batch, size_t n, int planes,
+                               const float* cg, float inv_n, hipStream_t s) {
+  hipLaunchKernelGGL(k_grad_reduce, dim3((unsigned)((n + 255) / 256), planes), dim3(256), 0, s, gitem,
+                     grad, batch, n, cg, inv_n);
+}
+
+static int adjoint_segment(bpmh_plan plan, int batch, int z_lo, int z_hi, float* g_,
+                           const float* u_seg_, long long u_seg_numel, const void* dn, int dn_kind,
+                           long long dn_numel, const float* H_, float unit_k, int absorb,
+                           float* grad_dn, float* gitem, long long work_numel, void* stream) {
   float2* g = (float2*)g_;
   const float2* u_seg = (const float2*)u_seg_;
   const float2* H = (const float2*)H_;
@@ -1885,6 +1877,22 @@ extern "C" int bpmh_adjoint_segment(bpmh_plan plan, int batch, int z_lo, int z_h
   ca.conj_h = 1;
 
   const size_t n = (size_t)n2 * comps;
+  // one launch when every step's per-item gradients fit the workspace
+  if (work_numel >= (long long)(nseg - 1) * batch * (long long)n) {
+    LoopCall call;
+    memset(&call, 0, sizeof call);
+    call.ra = ra;
+    call.ra.dn = (const char*)dn + (size_t)z_lo * n * sizeof(float);
+    call.ra.nz = nseg;
+    call.ca = ca;
+    const int rc = loop_run(plan, BPMH_MEAN_IGNORE, batch, nseg, call, s, true);
+    if (rc < 0) return rc;
+    if (rc == 1) {
+      launch_grad_reduce(gitem, grad_dn + (size_t)(z_lo + 1) * n, batch, n, nseg - 1, nullptr, 0.f, s);
+      HIP_TRY(hipGetLastError());
+      return BPMH_OK;
+    }
+  }
   for (int z = z_hi; z > z_lo; --z) {
     ra.z = z;
     ra.useg_z = z - z_lo;
@@ -1892,8 +1900,7 @@ extern "C" int bpmh_adjoint_segment(bpmh_plan plan, int batch, int z_lo, int z_h
     ra.screen = 1;
     ra.fwd_items = batch;
     row(ra, batch, s);
-    hipLaunchKernelGGL(k_grad_reduce, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, gitem,
-                       grad_dn + (size_t)z * n, batch, n);
+    launch_grad_reduce(gitem, grad_dn + (size_t)z * n, batch, n, 1, nullptr, 0.f, s);
     col0(ca, batch, s);
   }
   // back to real space: the gradient with respect to u[z_lo]
@@ -1904,6 +1911,38 @@ extern "C" int bpmh_adjoint_segment(bpmh_plan plan, int batch, int z_lo, int z_h
   row(ra, batch, s);
   HIP_TRY(hipGetLastError());
   return BPMH_OK;
+}
+
+extern "C" int bpmh_adjoint_segment(bpmh_plan plan, int batch, int z_lo, int z_hi, float* g,
+                                    const float* u_seg, long long u_seg_numel, const void* dn,
+                                    int dn_kind, long long dn_numel, const float* H, float unit_k,
+                                    int absorb, float* grad_dn, float* gitem, void* stream) {
+  return adjoint_segment(plan, batch, z_lo, z_hi, g, u_seg, u_seg_numel, dn, dn_kind, dn_numel, H,
+                         unit_k, absorb, grad_dn, gitem, 0, stream);
+}
+
+extern "C" int bpmh_adjoint_segment_work(bpmh_plan plan, int batch, int z_lo, int z_hi, int dn_kind,
+                                         long long* numel) {
+  if (!plan || !numel) return bpmh_set_error(BPMH_ERR_INVALID, "null argument");
+  if (batch < 1 || z_lo < 0 || z_hi < z_lo) return bpmh_set_error(BPMH_ERR_INVALID, "bad range");
+  const long long n = (long long)plan->nx * plan->ny * (dn_kind == BPMH_DN_C64 ? 2 : 1);
+  const bool loop = loop_adj_wanted(plan, BPMH_MEAN_IGNORE, batch, z_hi - z_lo + 1,
+                                    row_e_of(plan->nx, plan->row_v / kRowShapes),
+                                    col_e_of(plan->ny, plan->col_v / kColShapes));
+  *numel = n * batch * (loop ? z_hi - z_lo : 1);
+  return BPMH_OK;
+}
+
+extern "C" int bpmh_adjoint_segment_ws(bpmh_plan plan, int batch, int z_lo, int z_hi, float* g,
+                                       const float* u_seg, long long u_seg_numel, const void* dn,
+                                       int dn_kind, long long dn_numel, const float* H,
+                                       float unit_k, int absorb, float* grad_dn, float* work,
+                                       long long work_numel, void* stream) {
+  if (plan && batch >= 1 &&
+      work_numel < (long long)batch * plan->nx * plan->ny * (dn_kind == BPMH_DN_C64 ? 2 : 1))
+    return bpmh_set_error(BPMH_ERR_INVALID, "work holds less than one plane per item");
+  return adjoint_segment(plan, batch, z_lo, z_hi, g, u_seg, u_seg_numel, dn, dn_kind, dn_numel, H,
+                         unit_k, absorb, grad_dn, work, work_numel, stream);
 }
 
 // ----------------------------------------------------------------------------
@@ -1928,7 +1967,8 @@ struct WsegLayout {
   size_t wpart, dn0, fplane, useg, kseg, recc, recw, s1, s2, gitem, gd, cg, total;
 };
 
-static WsegLayout wseg_layout(int nx, int ny, int batch, int nseg, bool adjoint) {
+static WsegLayout wseg_layout(bpmh_plan plan, int batch, int nseg, bool adjoint) {
+  const int nx = plan->nx, ny = plan->ny;
   WsegLayout L;
   memset(&L, 0, sizeof L);
   size_t o = 0;
@@ -1948,30 +1988,20 @@ static WsegLayout wseg_layout(int nx, int ny, int batch, int nseg, bool adjoint)
     L.recw = take((S - 1) * B);
     L.s1 = take(B * ny);
     L.s2 = take(B * nx);
-    L.gitem = take(B * n2);
+    // screen gradients: of every step where they run as one launch, else of one
+    L.gitem = take(loop_size(plan) ? B * (S - 1) * n2 : B * n2);
     L.gd = take(B * n2);
-    L.cg = take(B);
+    L.cg = take(B * S);
   }
   L.total = o;
   return L;
-}
-
-// grad[i] += (sum_b cg[b]) / n over one plane: dL/ddn0 of a simple-mean step
-// spread over the plane it is the mean of (items summed in order)
-__global__ void k_add_mean_grad(float* __restrict__ grad, const float* __restrict__ cg, int batch,
-                                size_t n, float inv_n) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float c = 0.f;
-  for (int b = 0; b < batch; ++b) c += cg[b];
-  grad[i] += c * inv_n;
 }
 
 extern "C" int bpmh_mean_segment_work(bpmh_plan plan, int batch, int z_lo, int z_hi,
                                       int adjoint, long long* numel) {
   if (!plan || !numel) return bpmh_set_error(BPMH_ERR_INVALID, "null argument");
   if (batch < 1 || z_lo < 0 || z_hi < z_lo) return bpmh_set_error(BPMH_ERR_INVALID, "bad range");
-  *numel = (long long)wseg_layout(plan->nx, plan->ny, batch, z_hi - z_lo + 1, adjoint != 0).total;
+  *numel = (long long)wseg_layout(plan, batch, z_hi - z_lo + 1, adjoint != 0).total;
   return BPMH_OK;
 }
 
@@ -2001,7 +2031,7 @@ extern "C" int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z
              (long long)(z_hi + 1) * n2);
     return bpmh_set_error(BPMH_ERR_INVALID, msg);
   }
-  const WsegLayout L = wseg_layout(nx, ny, batch, nseg, adjoint);
+  const WsegLayout L = wseg_layout(plan, batch, nseg, adjoint);
   if (work_numel < (long long)L.total) {
     snprintf(msg, sizeof msg, "work holds %lld floats; this segment needs %lld", work_numel,
              (long long)L.total);
@@ -2060,12 +2090,28 @@ extern "C" int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z
   ca.wpart = (float2*)(work + L.wpart);
   ca.dn0_item = work + L.dn0;
 
+  int looped = 0;
+  {
+    LoopCall call;
+    memset(&call, 0, sizeof call);
+    call.ra = ra;
+    call.ca = ca;
+    if (adjoint) {
+      call.ca.kout = kseg;
+      call.ca.kout_bstride = (long long)(S - 1) * n2;
+      call.ca.rec_c = work + L.recc;
+      call.ca.rec_w = work + L.recw;
+      call.la.kout_zstride = n2;
+    }
+    looped = loop_run(plan, mean_mode, batch, nseg, call, s);
+    if (looped < 0) return looped;
+  }
   ra.z = 0;
   ra.fwd_items = batch;
-  row(ra, batch, s);
+  if (!looped) row(ra, batch, s);
   ra.inverse = 1;
   ra.screen = 1;
-  for (int z = 1; z < nseg; ++z) {
+  for (int z = 1; z < nseg && !looped; ++z) {
     ca.z = z;
     if (adjoint) {
       ca.kout = kseg + (size_t)(z - 1) * n2;
@@ -2128,15 +2174,31 @@ extern "C" int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z
   cb.s2part = work + L.s2;
   cb.s1part = work + L.s1;
   cb.gd_item = gd;
-  const unsigned red_blocks = (unsigned)((nn + 255) / 256);
+  {
+    LoopCall call;
+    memset(&call, 0, sizeof call);
+    call.ra = rb;
+    call.ra.fwd_items = 0;
+    call.ca = cb;
+    call.ca.uk = kseg;
+    call.ca.cz = work + L.recc;
+    call.ca.wz = work + L.recw;
+    const int rc = loop_run(plan, mean_mode, batch, nseg, call, s, true);
+    if (rc < 0) return rc;
+    if (rc == 1) {
+      launch_grad_reduce(gitem, grad_dn + (size_t)(z_lo + 1) * nn, batch, nn, nseg - 1,
+                         simple ? work + L.cg : nullptr, 1.f / (float)nn, s);
+      if (!simple) launch_grad_reduce(gd, grad_dn, batch, nn, 1, nullptr, 0.f, s);
+      HIP_TRY(hipGetLastError());
+      return BPMH_OK;
+    }
+  }
   for (int z = nseg - 1; z >= 1; --z) {
     rb.z = z;
     rb.useg_z = z;
     rb.inverse = z != nseg - 1;
     if (!simple) rb.dn0_item = work + L.recc + (size_t)(z - 1) * B;
     row(rb, batch, s);
-    hipLaunchKernelGGL(k_grad_reduce, dim3(red_blocks), dim3(256), 0, s, gitem,
-                       grad_dn + (size_t)(z_lo + z) * nn, batch, nn);
     hipLaunchKernelGGL(k_row_sums, dim3((unsigned)((B * ny + 3) / 4)), dim3(256), 0, s, gitem,
                        work + L.s1, (int)(B * ny), nx);
     cb.z = z;
@@ -2145,10 +2207,9 @@ extern "C" int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z
     cb.wz = work + L.recw + (size_t)(z - 1) * B;
     col3(cb, batch, s);
     col4(cb, batch, s);
-    if (simple)  // dn0 of this step is the mean of plane z: dL/ddn0 / N on every voxel
-      hipLaunchKernelGGL(k_add_mean_grad, dim3(red_blocks), dim3(256), 0, s,
-                         grad_dn + (size_t)(z_lo + z) * nn, (const float*)(work + L.cg), batch, nn,
-                         1.f / (float)nn);
+    // (simple: dn0 of this step is the mean of plane z, dL/ddn0 / N on every voxel)
+    launch_grad_reduce(gitem, grad_dn + (size_t)(z_lo + z) * nn, batch, nn, 1,
+                       simple ? work + L.cg : nullptr, 1.f / (float)nn, s);
   }
   rb.adjoint = 0;
   rb.screen = 0;
@@ -2157,7 +2218,7 @@ extern "C" int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z
   row(rb, batch, s);
   // the weight slice is slice 0 of the volume
   if (!simple)
-    hipLaunchKernelGGL(k_grad_reduce, dim3(red_blocks), dim3(256), 0, s, gd, grad_dn, batch, nn);
+    launch_grad_reduce(gd, grad_dn, batch, nn, 1, nullptr, 0.f, s);
   HIP_TRY(hipGetLastError());
   return BPMH_OK;
 }

@@ -90,6 +90,7 @@ struct LoopCall {
 
 template <int NX, int NY, int ER, int EC>
 struct LoopCfg {
+  static constexpr int POINTS = NX * NY;
   static constexpr int PTS = loop_points(NX, NY), SLOTS = loop_slots(NX, NY);
   static constexpr int E = EC;                  // points per thread
   static constexpr int TH = PTS / E;
@@ -182,6 +183,143 @@ BPMH_DEV int loop_nz(const RowArgs& ra, const LoopArgs& la, int field) {
   return nz;
 }
 
+// A work-group's place in its team, and the work that the team is at.
+template <class C>
+struct LoopTeam {
+  unsigned* flags;
+  int group, me;
+  unsigned xcd;
+  unsigned seq;          // last record seen
+  unsigned at;           // value of the flags once the phases so far are done
+  int lead_field, lead_z;
+  bool dead;             // a wait gave up
+  int M, field, z0, z1;  // members; the field and its planes z0 (done) to z1
+  bool whole, last;      // M == SLOTS; z1 is the field's last plane
+
+  // Registers this work-group; false when there is no team for it.
+  BPMH_DEV bool join(unsigned* sh) {
+    const LoopArgs& la = loop_args().la;
+    if (threadIdx.x == 0) {
+      const unsigned x = __builtin_amdgcn_s_getreg(20 | (3 << 11)) & (kLoopXcds - 1);  // XCC_ID
+      sh[0] = __hip_atomic_fetch_add(la.sync + 64 + 64 * x, 1u, __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_WORKGROUP);
+      sh[1] = x;
+    }
+    __syncthreads();
+    const unsigned rank = __builtin_amdgcn_readfirstlane(sh[0]);
+    xcd = __builtin_amdgcn_readfirstlane(sh[1]);
+    group = (int)(rank / C::SLOTS);
+    me = (int)(rank % C::SLOTS);
+    flags = la.sync + kLoopHead + ((size_t)xcd * la.teams + group) * kLoopTeamWords;
+    seq = at = 0;
+    lead_field = -1;
+    lead_z = 0;
+    dead = false;
+    return group < la.teams;
+  }
+
+  // Member 0, one wavefront: the previous chunk is complete, announce the next.
+  BPMH_DEV void announce() {
+    bool end = seq != 0 && !loop_wait(flags, C::SLOTS, at);
+    if (threadIdx.x != 0) return;
+    const LoopCall& call = loop_args();
+    // the first time, up to ~20 us for the team to come together
+    const __amdgpu_buffer_rsrc_t reg = loop_rsrc(call.la.sync, kLoopHead * 4);
+    int n = 0;
+    for (int k = 0; k < 64; ++k) {
+      n = (int)__builtin_amdgcn_raw_buffer_load_b32(reg, (64 + 64 * xcd) * 4, 0, kSc1) -
+          group * C::SLOTS;
+      asm volatile("" ::: "memory");
+      if (n >= C::SLOTS || seq != 0) break;
+      __builtin_amdgcn_s_sleep(8);
+    }
+    n = n > C::SLOTS ? C::SLOTS : (n < 1 ? 1 : n);
+    if (lead_field < 0 || lead_z >= loop_nz(call.ra, call.la, lead_field) - 1) {
+      lead_field = (int)__hip_atomic_fetch_add(call.la.sync, 1u, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+      lead_z = 0;
+    }
+    end |= lead_field >= call.la.batch;
+    const unsigned long long rec =
+        loop_pack(seq + 1, end, 31 - __clz(n), end ? 0 : lead_field, lead_z);
+    if (!end)
+      lead_z = min(lead_z + (n == C::SLOTS ? kLoopSteps : kLoopStepsPart),
+                   loop_nz(call.ra, call.la, lead_field) - 1);
+    publish(rec);
+  }
+  BPMH_DEV void publish(unsigned long long rec) {
+    __hip_atomic_store((unsigned long long*)(flags + 128), rec, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+
+  // The next chunk that counts this work-group in; false at the end.
+  BPMH_DEV bool next(unsigned long long* sh) {
+    if (threadIdx.x < 64) {
+      if (me == 0) announce();
+      const __amdgpu_buffer_rsrc_t team = loop_rsrc(flags, kLoopTeamWords * 4);
+      for (;;) {
+        const loop_u2 w = __builtin_amdgcn_raw_buffer_load_b64(team, 128 * 4, 0, kSc1);
+        asm volatile("" ::: "memory");
+        const unsigned hi = __builtin_amdgcn_readfirstlane(w.y);
+        const unsigned lo = __builtin_amdgcn_readfirstlane(w.x);
+        const unsigned s = hi >> 12;
+        if (s != seq) {
+          seq = s;
+          if (((hi >> 11) & 1) || me < (1 << ((hi >> 8) & 7))) {
+            if (threadIdx.x == 0) *sh = ((unsigned long long)hi << 32) | lo;
+            break;
+          }
+        }
+        __builtin_amdgcn_s_sleep(2);
+      }
+    }
+    __syncthreads();
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(*sh >> 32));
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)*sh);
+    if ((hi >> 11) & 1) return false;
+    seq = hi >> 12;
+    at = seq << 8;
+    M = 1 << ((hi >> 8) & 7);
+    field = (int)(((hi & 0xffu) << 12) | (lo >> 20));
+    z0 = (int)(lo & 0xfffffu);
+    whole = M == C::SLOTS;
+    const LoopCall& call = loop_args();
+    const int nz = loop_nz(call.ra, call.la, field);
+    z1 = min(z0 + (whole ? kLoopSteps : kLoopStepsPart), nz - 1);
+    last = z1 == nz - 1;
+    return true;
+  }
+
+  // Before a phase: every slot of the phase before it is done.  (The first
+  // phase of a chunk: the leader saw that before it wrote the record.)
+  BPMH_DEV void enter(bool first, unsigned* sh) {
+    if (first) return;
+    if (threadIdx.x < 64) {
+      const bool ok = loop_wait(flags, C::SLOTS, at);
+      if (threadIdx.x == 0) sh[0] = ok;
+    }
+    __syncthreads();
+    dead |= __builtin_amdgcn_readfirstlane(sh[0]) == 0;
+  }
+  // Slot s of the phase is done (the caller adds 1 to `at` after its slots).
+  BPMH_DEV void leave(int s) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0)
+      __hip_atomic_store(flags + s, at + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+
+  // A wait gave up (a member of the team stopped): marks this slot's rows of
+  // the plane; the leader ends the team.
+  BPMH_DEV void give_up(float2* planes) {
+    const __amdgpu_buffer_rsrc_t rp = loop_rsrc(planes + (size_t)field * C::POINTS, C::POINTS * 8);
+    const float nan = __uint_as_float(0x7fc00000u);
+    for (int i = threadIdx.x; i < C::PTS; i += C::TH)
+      loop_st(rp, i * 8, me * C::PTS * 8, make_float2(nan, nan));
+    if (me == 0 && threadIdx.x == 0) publish(loop_pack(seq + 1, true, 0, 0, 0));
+  }
+};
+
 // row_screen of a forward step, the same operations, for a kernel that keeps
 // state in registers around it: one element after another, the taper from a
 // table in LDS, and the rare or heavy forms (a phase beyond pi/4 in any lane
@@ -267,25 +405,8 @@ k_loop(LoopCall) {
   __shared__ float sh_acc[HKEEP ? 1 : C::PTS];  // a complete team's running |u|^2 sums, [element][thread]
   const int tid0 = threadIdx.x;
 
-  int group, me;
-  unsigned* flags;
-  unsigned xcd;
-  {
-    const LoopArgs& la = loop_args().la;
-    if (tid0 == 0) {
-      const unsigned x = __builtin_amdgcn_s_getreg(20 | (3 << 11)) & (kLoopXcds - 1);  // XCC_ID
-      sh_u[0] = __hip_atomic_fetch_add(la.sync + 64 + 64 * x, 1u, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_WORKGROUP);
-      sh_u[1] = x;
-    }
-    __syncthreads();
-    const unsigned rank = __builtin_amdgcn_readfirstlane(sh_u[0]);
-    xcd = __builtin_amdgcn_readfirstlane(sh_u[1]);
-    group = (int)(rank / SLOTS);
-    me = (int)(rank % SLOTS);
-    if (group >= la.teams) return;
-    flags = la.sync + kLoopHead + ((size_t)xcd * la.teams + group) * kLoopTeamWords;
-  }
+  LoopTeam<C> tm;
+  if (!tm.join(sh_u)) return;
   {
     const int w = min(loop_args().ra.absorb, HALF);
     for (int d = tid0; d < w; d += C::TH) sh_taper[d] = taper_factor(d, loop_args().ra.absorb);
@@ -300,96 +421,10 @@ k_loop(LoopCall) {
   float2 v[EC];       // columns (kept from phase A to phase B of the weighted mean)
   float dpre[QR][ER];     // dn of the next row phase (real dn)
 
-  unsigned seq = 0;       // last record seen
-  int lead_field = -1, lead_z = 0;
-  unsigned at = 0;        // value of the flags once the phases so far are done
-  for (;;) {
-    if (tid0 < 64) {
-      if (me == 0) {
-        bool end = seq != 0 && !loop_wait(flags, SLOTS, at);
-        if (tid0 == 0) {
-          const LoopCall& call = loop_args();
-          // the first time, up to ~20 us for the team to come together
-          const __amdgpu_buffer_rsrc_t reg = loop_rsrc(call.la.sync, kLoopHead * 4);
-          int n = 0;
-          for (int k = 0; k < 64; ++k) {
-            n = (int)__builtin_amdgcn_raw_buffer_load_b32(reg, (64 + 64 * xcd) * 4, 0, kSc1) -
-                group * SLOTS;
-            asm volatile("" ::: "memory");
-            if (n >= SLOTS || seq != 0) break;
-            __builtin_amdgcn_s_sleep(8);
-          }
-          n = n > SLOTS ? SLOTS : (n < 1 ? 1 : n);
-          if (lead_field < 0 || lead_z >= loop_nz(call.ra, call.la, lead_field) - 1) {
-            lead_field = (int)__hip_atomic_fetch_add(call.la.sync, 1u, __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT);
-            lead_z = 0;
-          }
-          end |= lead_field >= call.la.batch;
-          const unsigned long long rec =
-              loop_pack(seq + 1, end, 31 - __clz(n), end ? 0 : lead_field, lead_z);
-          if (!end)
-            lead_z = min(lead_z + (n == SLOTS ? kLoopSteps : kLoopStepsPart),
-                         loop_nz(call.ra, call.la, lead_field) - 1);
-          __hip_atomic_store((unsigned long long*)(flags + 128), rec, __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_WORKGROUP);
-        }
-      }
-      // the next record that counts this work-group in, or the end
-      const __amdgpu_buffer_rsrc_t team = loop_rsrc(flags, kLoopTeamWords * 4);
-      for (;;) {
-        const loop_u2 w = __builtin_amdgcn_raw_buffer_load_b64(team, 128 * 4, 0, kSc1);
-        asm volatile("" ::: "memory");
-        const unsigned hi = __builtin_amdgcn_readfirstlane(w.y);
-        const unsigned lo = __builtin_amdgcn_readfirstlane(w.x);
-        const unsigned s = hi >> 12;
-        if (s != seq) {
-          seq = s;
-          if (((hi >> 11) & 1) || me < (1 << ((hi >> 8) & 7))) {
-            if (tid0 == 0) sh_rec = ((unsigned long long)hi << 32) | lo;
-            break;
-          }
-        }
-        __builtin_amdgcn_s_sleep(2);
-      }
-    }
-    __syncthreads();
-    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(sh_rec >> 32));
-    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)sh_rec);
-    if ((hi >> 11) & 1) return;
-    seq = hi >> 12;
-    const int M = 1 << ((hi >> 8) & 7);
-    const int field = (int)(((hi & 0xffu) << 12) | (lo >> 20)), z0 = (int)(lo & 0xfffffu);
-    const bool whole = M == SLOTS;
-    int z1;
-    bool last;              // the field's last plane is in this chunk
-    {
-      const LoopCall& call = loop_args();
-      const int nz = loop_nz(call.ra, call.la, field);
-      z1 = min(z0 + (whole ? kLoopSteps : kLoopStepsPart), nz - 1);
-      last = z1 == nz - 1;
-    }
-    at = seq << 8;
-    bool dead = false;
-
-    // Before a phase: every slot of the phase before it is done.  (The first
-    // phase of a chunk: the leader saw that before it wrote the record.)
-    auto enter = [&](bool first) __attribute__((always_inline)) {
-      if (!first) {
-        if (tid0 < 64) {
-          const bool ok = loop_wait(flags, SLOTS, at);
-          if (tid0 == 0) sh_u[0] = ok;
-        }
-        __syncthreads();
-        dead |= __builtin_amdgcn_readfirstlane(sh_u[0]) == 0;
-      }
-    };
-    auto leave = [&](int s) __attribute__((always_inline)) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
-      if (tid0 == 0)
-        __hip_atomic_store(flags + s, at + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    };
+  while (tm.next(&sh_rec)) {
+    const int field = tm.field, me = tm.me, M = tm.M;
+    const int z0 = tm.z0, z1 = tm.z1;
+    const bool whole = tm.whole, last = tm.last;
     auto load_h = [&](float2 (&hv)[EC], const ColArgs& ca, int s, int tid) __attribute__((always_inline)) {
       const int cl = tid % C::LC, tc = tid / C::LC;
       const int x = s * C::LC + cl;
@@ -472,8 +507,8 @@ k_loop(LoopCall) {
       const RowArgs& ra = loop_args().ra;
       Twiddles<NX, ER> tw;
       tw.load(loop_opaque(tid0) % TR, ra.tw);
-      enter(first);
-      if (dead) return;
+      tm.enter(first, sh_u);
+      if (tm.dead) return;
       const __amdgpu_buffer_rsrc_t rp = loop_rsrc(ra.plane + (size_t)field * NX * NY, NX * NY * 8);
       const bool screened = z > 0 && ra.dn_kind != BPMH_DN_NONE;
       const bool end = last && z == z1;  // the field's last plane: no forward transform
@@ -524,9 +559,9 @@ k_loop(LoopCall) {
           for (int m = 0; m < ER; ++m)
             loop_st(rp, off, ((s * C::LR + q * C::LRP) * NX + m * TR) * 8, u[q][m]);
         }
-        leave(s);
+        tm.leave(s);
       }
-      at += 1;
+      tm.at += 1;
     };
 
     // static or per-plane propagator: FFT_y, H, IFFT_y
@@ -536,8 +571,8 @@ k_loop(LoopCall) {
       const ColArgs& ca = call.ca;
       Twiddles<NY, EC> tw;
       tw.load(loop_opaque(tid0) / C::LC, ca.tw);
-      enter(first);
-      if (dead) return;
+      tm.enter(first, sh_u);
+      if (tm.dead) return;
       const __amdgpu_buffer_rsrc_t rp = loop_rsrc(ca.plane + (size_t)field * NX * NY, NX * NY * 8);
       const bool screened = call.ra.dn_kind != BPMH_DN_NONE;
       for (int s = me; s < SLOTS; s += M) {
@@ -564,9 +599,9 @@ k_loop(LoopCall) {
         if (ca.sw) col_scatter<NY, EC>(ca, z, field, x, tc, ln, v);
         line_fft<NY, EC, true, CL>(v, ln, tc, tw);
         store_cols(v, rp, s, cl, tc);
-        leave(s);
+        tm.leave(s);
       }
-      at += 1;
+      tm.at += 1;
     };
 
     // weighted mean: A (FFT_y, per-column sums), B (dn0, H(n0 + dn0), IFFT_y);
@@ -576,8 +611,8 @@ k_loop(LoopCall) {
       const ColArgs& ca = call.ca;
       Twiddles<NY, EC> tw;
       tw.load(loop_opaque(tid0) / C::LC, ca.tw);
-      enter(first);
-      if (dead) return;
+      tm.enter(first, sh_u);
+      if (tm.dead) return;
       const __amdgpu_buffer_rsrc_t rp = loop_rsrc(ca.plane + (size_t)field * NX * NY, NX * NY * 8);
       const bool screened = call.ra.dn_kind != BPMH_DN_NONE;
       for (int s = me; s < SLOTS; s += M) {
@@ -594,11 +629,11 @@ k_loop(LoopCall) {
         if (tc == 0) ca.wpart[(size_t)field * NX + s * C::LC + cl] = sums;
         if (ca.kout) record(v, call, s, z, cl, tc);
         if (!whole) store_cols(v, rp, s, cl, tc);
-        leave(s);
+        tm.leave(s);
       }
-      at += 1;
-      enter(false);
-      if (dead) return;
+      tm.at += 1;
+      tm.enter(false, sh_u);
+      if (tm.dead) return;
       // dn0 in the fixed order of weighted_dn0_group
       if (tid0 < 64) {
         const __amdgpu_buffer_rsrc_t rw = loop_rsrc(ca.wpart + (size_t)field * NX, NX * 8);
@@ -642,31 +677,22 @@ k_loop(LoopCall) {
         if (ca.sw) col_scatter<NY, EC>(ca, z, field, x, tc, ln, v);
         line_fft<NY, EC, true, CL>(v, ln, tc, tw);
         store_cols(v, rp, s, cl, tc);
-        leave(s);
+        tm.leave(s);
       }
-      at += 1;
+      tm.at += 1;
     };
 
     // plane 0 has a row phase alone (outputs of u0, FFT_x)
     const int zb = z0 == 0 ? 0 : z0 + 1;
-    for (int z = zb; z <= z1 && !dead; ++z) {
+    for (int z = zb; z <= z1 && !tm.dead; ++z) {
       if (z > 0) {
         if constexpr (MODE == BPMH_MEAN_WEIGHTED) weighted_phases(z, z == zb);
         else col_phase(z, z == zb);
       }
-      if (!dead) row_phase(z, z == 0);
+      if (!tm.dead) row_phase(z, z == 0);
     }
-    if (dead) {
-      // a wait gave up (a member of the team stopped): mark this slot's rows
-      // and leave; the leader ends the team
-      const LoopCall& call = loop_args();
-      const __amdgpu_buffer_rsrc_t rp = loop_rsrc(call.ra.plane + (size_t)field * NX * NY, NX * NY * 8);
-      const float nan = __uint_as_float(0x7fc00000u);
-      for (int i = tid0; i < C::LR * NX; i += C::TH)
-        loop_st(rp, i * 8, me * C::LR * NX * 8, make_float2(nan, nan));
-      if (me == 0 && tid0 == 0)
-        __hip_atomic_store((unsigned long long*)(flags + 128), loop_pack(seq + 1, true, 0, 0, 0),
-                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (tm.dead) {
+      tm.give_up(loop_args().ra.plane);
       return;
     }
   }

@@ -265,6 +265,15 @@ BPMH_DEV float2 c_mul_fused(float2 a, float2 b) {
   return make_float2(fmaf(a.x, b.x, -f_mul(a.y, b.y)), fmaf(a.x, b.y, f_mul(a.y, b.x)));
 }
 
+// a*conj(b) likewise.
+BPMH_DEV float2 c_mulc_fused(float2 a, float2 b) { return c_mul_fused(a, make_float2(b.x, -b.y)); }
+
+// conj(g) u: its imaginary and real part are the screen gradients in Re dn
+// and Im dn (times k0 dz).
+BPMH_DEV float2 adjoint_pair(float2 g, float2 u) {
+  return make_float2(fmaf(g.x, u.x, f_mul(g.y, u.y)), fmaf(g.x, u.y, -f_mul(g.y, u.x)));
+}
+
 // Taper 1/2 (1 - cos(pi dist / width)) of a voxel `dist` from the border.
 BPMH_DEV float taper_factor(int dist, int width) {
   const float arg = f_div(f_mul(BPMH_PI_F, (float)dist), (float)width);
@@ -292,11 +301,10 @@ BPMH_DEV void row_screen(const RowArgs& a, int b, int y, int t, float dn0, const
       if (ADJ && a.adjoint) {
         // u = s v with s = e^{k Im dn} e^{-i k Re dn}: dL/dRe dn = k Im(conj(G) u),
         // dL/dIm dn = k Re(conj(G) u), and G_v = conj(s) G
-        const float2 w = make_float2(v[m].x * ua[m].x + v[m].y * ua[m].y,
-                                     v[m].x * ua[m].y - v[m].y * ua[m].x);
+        const float2 w = adjoint_pair(v[m], ua[m]);
         reinterpret_cast<float2*>(a.gitem)[((size_t)b * a.ny + y) * NX + x] =
             make_float2(a.unit_k * w.y, a.unit_k * w.x);
-        v[m] = c_mulc(v[m], make_float2(mag * c, mag * s));
+        v[m] = c_mulc_fused(v[m], make_float2(mag * c, mag * s));
       } else {
         v[m] = c_mul_fused(v[m], make_float2(mag * c, mag * s));
       }
@@ -306,8 +314,8 @@ BPMH_DEV void row_screen(const RowArgs& a, int b, int y, int t, float dn0, const
       sincos_fast(ph, &s, &c);
       float2 r;
       if (ADJ && a.adjoint) {
-        a.gitem[((size_t)b * a.ny + y) * NX + x] = a.unit_k * (v[m].x * ua[m].y - v[m].y * ua[m].x);
-        r = c_mulc(v[m], make_float2(c, s));
+        a.gitem[((size_t)b * a.ny + y) * NX + x] = a.unit_k * adjoint_pair(v[m], ua[m]).y;
+        r = c_mulc_fused(v[m], make_float2(c, s));
       } else {
         r = c_mul_fused(v[m], make_float2(c, s));
       }
@@ -449,4 +457,70 @@ BPMH_DEV void col_scatter(const ColArgs& a, int z, int b, int x, int t, float2* 
   acc = column_sum2<T>(acc, line, t);
   if (t == 0) a.spart[((size_t)b * a.nz + z) * a.nx + x] = acc;
   __syncthreads();  // the line is the inverse transform's exchange buffer
+}
+
+// Mean-corrected adjoint, one column: H and beta = the axial wavenumber (0
+// where nothing propagates) of every row, as col_h_fly; and the column's sum
+// of Im(conj(X) H U) / beta (valid in every thread).
+template <int NY, int E>
+BPMH_DEV void col_hb_fly(float kx2, float an, float dy, float dz, int t, float2* line, float2 (&h)[E],
+                         float (&bt)[E]) {
+  constexpr int T = NY / E;
+#pragma unroll
+  for (int m = 0; m < E / 2; ++m)
+    h[m] = prop_f32_beta(kx2, kcomp2_f32(t + m * T, NY, dy), an, dz, &bt[m]);
+  if (t == 0) h[E / 2] = prop_f32_beta(kx2, kcomp2_f32(NY / 2, NY, dy), an, dz, &bt[E / 2]);
+  __syncthreads();  // earlier users of the line are done with it
+#pragma unroll
+  for (int m = 0; m < E / 2; ++m) {
+    line[m * T + t] = h[m];
+    line[NY / 2 + m * T + t] = make_float2(bt[m], 0.f);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = E / 2; m < E; ++m) {
+    if (t == 0) {
+      if (m > E / 2) {
+        h[m] = h[E - m];
+        bt[m] = bt[E - m];
+      }
+    } else {
+      h[m] = line[(E - 1 - m) * T + T - t];
+      bt[m] = line[NY / 2 + (E - 1 - m) * T + T - t].x;
+    }
+  }
+}
+
+template <int NY, int E>
+BPMH_DEV float col_beta_sum(const float2 (&v)[E], const float2 (&h)[E], const float2 (&uv)[E],
+                            const float (&bt)[E], int t, float2* line) {
+  float acc = 0.f;  // (column_sum2 waits for every reader of the line)
+#pragma unroll
+  for (int m = 0; m < E; ++m) {
+    if (bt[m] > 0.f) {
+      const float2 hu = c_mul_fused(h[m], uv[m]);
+      acc += fmaf(v[m].x, hu.y, -f_mul(v[m].y, hu.x)) / bt[m];
+    }
+  }
+  return column_sum2<NY / E>(make_float2(acc, 0.f), line, t).x;
+}
+
+// dL/ddn0 = -sum_x (screen gradient) + dz (n0+dn0) k0^2 / N sum_k Im(conj(X) H U)/beta
+BPMH_DEV float adjoint_cgrad(float s1, float s2, float dz, float n, float k0, float n_pts) {
+  const float c = f_div(f_mul(f_mul(f_mul(dz, n), k0), k0), n_pts);
+  return fmaf(c, s2, -s1);
+}
+
+// dn0 = sum|U| d / sum|U| depends on U through |U|: the k-space gradient v
+// gains dL/ddn0 (d - dn0) / W * U/|U| (times N: X is N G_V); returns
+// dL/dd = dL/ddn0 |U| / W.
+BPMH_DEV float adjoint_weight_term(float2& v, float2 u, float d, float dn0, float cgrad, float inv_w,
+                                   float n_pts) {
+  const float au = hypotf(u.x, u.y);
+  if (au > 0.f) {
+    const float coef = f_div(f_mul(f_mul(f_mul(n_pts, cgrad), f_sub(d, dn0)), inv_w), au);
+    v.x = fmaf(coef, u.x, v.x);
+    v.y = fmaf(coef, u.y, v.y);
+  }
+  return f_mul(f_mul(cgrad, au), inv_w);
 }

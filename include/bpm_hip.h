@@ -247,6 +247,18 @@ int bpmh_adjoint_segment(bpmh_plan plan, int batch, int z_lo, int z_hi, float* g
                          long long dn_numel, const float* H, float unit_k, int absorb,
                          float* grad_dn, float* gitem, void* stream);
 
+/* bpmh_adjoint_segment with a workspace of work_numel floats instead of
+ * gitem: with bpmh_adjoint_segment_work's count (at the plan's launch shapes; the
+ * screen gradients of every step and item where the segment runs as one
+ * launch, bpmh_plan_set_loop) that is one launch and a reduction; one plane per
+ * item is the least it takes.  The results are the same bits. */
+int bpmh_adjoint_segment_work(bpmh_plan plan, int batch, int z_lo, int z_hi, int dn_kind,
+                              long long* numel);
+int bpmh_adjoint_segment_ws(bpmh_plan plan, int batch, int z_lo, int z_hi, float* g,
+                            const float* u_seg, long long u_seg_numel, const void* dn, int dn_kind,
+                            long long dn_numel, const float* H, float unit_k, int absorb,
+                            float* grad_dn, float* work, long long work_numel, void* stream);
+
 /* The differentiable form under bpm_3d's mean corrections, one segment
  * z_lo..z_hi of a float32 dn volume (nz, ny, nx) shared by the batch
  * (dn_numel elements, at least (z_hi+1)*ny*nx); n0, k0, dx, dy, dz, unit_k,
