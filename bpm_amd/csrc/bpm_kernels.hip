@@ -14,6 +14,7 @@
 // default mean_mode "weighted" of bpm_3d needs the k-space reduction of
 // bpm_3d.py:302-303 before H, so its column pass is split in two (A: FFT_y
 // and per-column partial sums; B: H(n0+dn0) and IFFT_y).
+#include "items.hpp"
 #include "loop_adj.hpp"
 
 #include <cmath>
@@ -1065,7 +1066,7 @@ static bool loop_size(bpmh_plan plan) {
 // 1024-thread groups (512 x 256 at 4.4, batch 50: 83 against 70 us per step);
 // at 512^2, 32 CUs are too few for a field alone (batch 1: 14.0 against 12.5)
 // and only 8.8 fits two groups a CU (batch 2: 14.3 against 15.7; 16: 27.8
-// against 48; at 4.8 and batch 17 52.7 against 49.5).
+// against 40; at 4.8 and batch 17 52.7 against 49.5).
 static bool loop_wanted(bpmh_plan plan, int batch, int nz, int er, int ec) {
   const int nx = plan->nx, ny = plan->ny;
   if (plan->loop_mode == 1 || nz < 2 || !loop_size(plan)) return false;
@@ -1082,11 +1083,11 @@ static bool loop_wanted(bpmh_plan plan, int batch, int nz, int er, int ec) {
 // more than one wavefront; the reduction's grid has a block row per plane.
 // Without a mean correction a step is short beside the forward planes it reads
 // and the screen gradients it writes, so from 512 x 256 on only while the
-// teams take the batch in one round (512^2 at 8.8, batch 8: 34 against 39 us
-// per step, 16: 68 against 59; 512 x 256, batch 1: 16.3 against 15.7, 16: 33
-// against 38, 50: 112 against 88; 256^2, batch 50: 37 against 55).  With one
+// teams take the batch in one round (512^2 at 8.8, batch 8: 34.2 against 34.5
+// us per step, 16: 68 against 53; 512 x 256, batch 1: 16.3 against 15.7, 16: 33
+// against 35, 50: 112 against 80; 256^2, batch 50: 37 against 55).  With one
 // it is 1.1 to 2.1 times faster throughout (512^2 at 8.8, batch 8: 81 against
-// 120, 50: 544 against 622).
+// 116, 50: 546 against 591).
 static bool loop_adj_wanted(bpmh_plan plan, int mode, int batch, int nz, int er, int ec) {
   const long long pts = (long long)plan->nx * plan->ny;
   if (!loop_wanted(plan, batch, nz, er, ec) || plan->nx / er > 64 || nz > 65536) return false;
@@ -1149,6 +1150,77 @@ extern "C" int bpmh_plan_set_loop(bpmh_plan p, int mode) {
   if (mode < 0 || mode > 3) return bpmh_set_error(BPMH_ERR_INVALID, "loop mode is 0 to 3");
   p->loop_mode = mode;
   return BPMH_OK;
+}
+
+// ----------------------------------------------------------------------------
+// passes of several items per work-group (items.hpp)
+// ----------------------------------------------------------------------------
+// They run from kItemsRows/kItemsCols points of a call on.  us per step with
+// the one-item passes / with these (each pass alone; running sum kept):
+//   1024^2  batch 2: 36.0 / 34.4 (rows 35.4, columns 34.4)
+//           batch 3: 49.0 / 40.5 (44.1, 44.7);  4: 62.1 / 45.9;  16: 191 / 139
+//   2048^2  batch 1: 81.1 / 63.7 (73.5, 72.3);  4: 274 / 164
+//   512 x 1024  batch 16: 118 / 80;   1024 x 512  batch 16: 90 / 69
+// Below, their registers leave too few wavefronts to hide a short call's
+// latencies: rows of 2 M points 33.4 against 32.2 (2048 x 64, batch 16), of
+// 1 M 24.3 against 21.7 (1024^2, batch 1); columns of 1 M points 27.9 against
+// 24.9 (256 x 2048, batch 2).
+constexpr long long kItemsRows = 5 << 19, kItemsCols = 2 << 20;
+constexpr long long kItemsThreads = 256 << 10;  // 16 wavefronts a CU
+
+// Items per work-group: as many as leave 16 wavefronts a CU, at most 8.
+static int items_per(long long threads, int batch) {
+  const long long most = threads / kItemsThreads;
+  const int per = (int)(most < 1 ? 1 : (most > 8 ? 8 : most));
+  const int chunks = (batch + per - 1) / per;
+  return (batch + chunks - 1) / chunks;
+}
+
+template <int NX>
+static void launch_row_items(const RowArgs& a, int batch, hipStream_t s) {
+  constexpr int E = row_e_of(NX, 0), T = NX / E, LINES = T >= 256 ? 1 : 256 / T;
+  const bool shared = a.ngroups == 0 && a.dn_bstride == 0 && a.dn0_mode != BPMH_MEAN_WEIGHTED;
+  const int per = shared || !a.screen ? items_per((long long)batch * a.ny * T, batch) : 1;
+  const dim3 g(a.ny / LINES, (batch + per - 1) / per), b(T * LINES);
+  if (a.adjoint) hipLaunchKernelGGL((k_row_items<NX, E, LINES, E == 4 ? 5 : 3, true>), g, b, 0, s, a, batch, per);
+  else hipLaunchKernelGGL((k_row_items<NX, E, LINES, E == 4 ? 5 : 3, false>), g, b, 0, s, a, batch, per);
+}
+template <int NY>
+static void launch_col_items(const ColArgs& a, int batch, hipStream_t s) {
+  constexpr int E = col_e_of(NY, 0), T = NY / E, LC = T >= 128 ? 4 : 8;
+  const int per = items_per((long long)batch * a.nx * T, batch);
+  const dim3 g(a.nx / LC, (batch + per - 1) / per), b(T * LC);
+  if (a.hmode == 0) hipLaunchKernelGGL((k_col_items<NY, E, LC, 4, false>), g, b, 0, s, a, batch, per);
+  else hipLaunchKernelGGL((k_col_items<NY, E, LC, 4, true>), g, b, 0, s, a, batch, per);
+}
+
+static void run_row(bpmh_plan plan, row_fn row, const RowArgs& a, int batch, hipStream_t s) {
+  const int nx = plan->nx;
+  if ((nx == 512 || nx == 1024 || nx == 2048) && (long long)batch * nx * plan->ny >= kItemsRows &&
+      (!a.adjoint || a.screen)) {
+    RowArgs r = a;
+    r.tw = plan->tw_x[0];
+    if (nx == 512) launch_row_items<512>(r, batch, s);
+    else if (nx == 1024) launch_row_items<1024>(r, batch, s);
+    else launch_row_items<2048>(r, batch, s);
+  } else {
+    row(a, batch, s);
+  }
+}
+
+// Column passes with H of a table or of n_eff[z].
+static void run_col(bpmh_plan plan, col_fn col, const ColArgs& a, int batch, hipStream_t s) {
+  const int ny = plan->ny;
+  if ((ny == 512 || ny == 1024 || ny == 2048) && (long long)batch * ny * plan->nx >= kItemsCols &&
+      !a.sw) {
+    ColArgs r = a;
+    r.tw = plan->tw_y[0];
+    if (ny == 512) launch_col_items<512>(r, batch, s);
+    else if (ny == 1024) launch_col_items<1024>(r, batch, s);
+    else launch_col_items<2048>(r, batch, s);
+  } else {
+    col(a, batch, s);
+  }
 }
 
 // Enqueue (or capture and replay) the whole z-loop of one call on stream s.
@@ -1275,7 +1347,7 @@ static int prop_run(bpmh_plan plan, const PropCall& c, const StepScratch& sc, hi
   ra.inverse = 0;
   ra.screen = 0;
   ra.fwd_items = nz > 1 ? batch : 0;
-  timed(TK_ROW, [&] { row(ra, batch, s); });
+  timed(TK_ROW, [&] { run_row(plan, row, ra, batch, s); });
   ra.acc_init = 0;
   ra.inverse = 1;
   ra.screen = c.dn_kind != BPMH_DN_NONE;
@@ -1285,11 +1357,11 @@ static int prop_run(bpmh_plan plan, const PropCall& c, const StepScratch& sc, hi
       timed(TK_COL_A, [&] { colA(ca, batch, s); });
       timed(TK_COL_B, [&] { colB(ca, batch, s); });
     } else {
-      timed(TK_COL, [&] { col0(ca, batch, s); });
+      timed(TK_COL, [&] { run_col(plan, col0, ca, batch, s); });
     }
     ra.z = z;
     ra.fwd_items = z < nz - 1 ? batch : 0;
-    timed(TK_ROW, [&] { row(ra, batch, s); });
+    timed(TK_ROW, [&] { run_row(plan, row, ra, batch, s); });
   }
   if (c.out_scat) {
     hipLaunchKernelGGL(k_scatter_final, dim3((nz + 63) / 64, batch), dim3(64), 0, s, sc.spart,
@@ -1541,7 +1613,7 @@ extern "C" int bpmh_propagate(bpmh_plan plan, int batch, int nz, float* plane, c
 // ----------------------------------------------------------------------------
 // The launches per pass of a ragged batch: group g of items[g] fields, depth
 // nzs[g]; events as in bpmh_propagate_groups.
-static int groups_launches(row_fn row, col_fn col, RowArgs ra, ColArgs ca, int dn_kind, int n_groups,
+static int groups_launches(bpmh_plan plan, row_fn row, col_fn col, RowArgs ra, ColArgs ca, int dn_kind, int n_groups,
                            const int* items, const int* nzs, int total, void** group_done,
                            hipStream_t s) {
   // items still propagating at plane z (and, for the forward transform, past
@@ -1563,7 +1635,7 @@ static int groups_launches(row_fn row, col_fn col, RowArgs ra, ColArgs ca, int d
   ra.inverse = 0;
   ra.screen = 0;
   ra.fwd_items = items_deeper(1);
-  row(ra, total, s);
+  run_row(plan, row, ra, total, s);
   int rc = mark_done(0);
   if (rc) return rc;
   ra.acc_init = 0;
@@ -1572,10 +1644,10 @@ static int groups_launches(row_fn row, col_fn col, RowArgs ra, ColArgs ca, int d
   for (int z = 1; z < nzs[0]; ++z) {
     const int active = items_deeper(z);
     ca.z = z;
-    col(ca, active, s);
+    run_col(plan, col, ca, active, s);
     ra.z = z;
     ra.fwd_items = items_deeper(z + 1);
-    row(ra, active, s);
+    run_row(plan, row, ra, active, s);
     rc = mark_done(z);
     if (rc) return rc;
   }
@@ -1666,7 +1738,7 @@ extern "C" int bpmh_propagate_groups(bpmh_plan plan, int n_groups, const int* it
       if (group_done && group_done[0]) HIP_TRY(hipEventRecord((hipEvent_t)group_done[0], s));
       return BPMH_OK;
     }
-    return groups_launches(row, col, ra, ca, dn_kind, n_groups, items, nzs, total, group_done, s);
+    return groups_launches(plan, row, col, ra, ca, dn_kind, n_groups, items, nzs, total, group_done, s);
   }
   const size_t dn_size = dn_kind == BPMH_DN_F16 ? 2 : (dn_kind == BPMH_DN_C64 ? 8 : 4);
   int g = n_groups;
@@ -1686,7 +1758,7 @@ extern "C" int bpmh_propagate_groups(bpmh_plan plan, int n_groups, const int* it
   }
   if (g == 0) return BPMH_OK;
   // the groups left (all of them, unless a synchronisation buffer ran out)
-  return groups_launches(row, col, ra, ca, dn_kind, g, items, nzs, total, group_done, s);
+  return groups_launches(plan, row, col, ra, ca, dn_kind, g, items, nzs, total, group_done, s);
 }
 
 // ----------------------------------------------------------------------------
@@ -1899,16 +1971,16 @@ static int adjoint_segment(bpmh_plan plan, int batch, int z_lo, int z_hi, float*
     ra.inverse = z != z_hi;
     ra.screen = 1;
     ra.fwd_items = batch;
-    row(ra, batch, s);
+    run_row(plan, row, ra, batch, s);
     launch_grad_reduce(gitem, grad_dn + (size_t)z * n, batch, n, 1, nullptr, 0.f, s);
-    col0(ca, batch, s);
+    run_col(plan, col0, ca, batch, s);
   }
   // back to real space: the gradient with respect to u[z_lo]
   ra.adjoint = 0;
   ra.screen = 0;
   ra.inverse = 1;
   ra.fwd_items = 0;
-  row(ra, batch, s);
+  run_row(plan, row, ra, batch, s);
   HIP_TRY(hipGetLastError());
   return BPMH_OK;
 }
@@ -2108,7 +2180,7 @@ extern "C" int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z
   }
   ra.z = 0;
   ra.fwd_items = batch;
-  if (!looped) row(ra, batch, s);
+  if (!looped) run_row(plan, row, ra, batch, s);
   ra.inverse = 1;
   ra.screen = 1;
   for (int z = 1; z < nseg && !looped; ++z) {
@@ -2120,14 +2192,14 @@ extern "C" int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z
       ca.rec_w = work + L.recw + (size_t)(z - 1) * B;
     }
     if (simple) {
-      col0(ca, batch, s);
+      run_col(plan, col0, ca, batch, s);
     } else {
       colA(ca, batch, s);
       colB(ca, batch, s);
     }
     ra.z = z;
     ra.fwd_items = z < nseg - 1 ? batch : 0;
-    row(ra, batch, s);
+    run_row(plan, row, ra, batch, s);
   }
   if (!adjoint) {
     HIP_TRY(hipGetLastError());
@@ -2198,7 +2270,7 @@ extern "C" int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z
     rb.useg_z = z;
     rb.inverse = z != nseg - 1;
     if (!simple) rb.dn0_item = work + L.recc + (size_t)(z - 1) * B;
-    row(rb, batch, s);
+    run_row(plan, row, rb, batch, s);
     hipLaunchKernelGGL(k_row_sums, dim3((unsigned)((B * ny + 3) / 4)), dim3(256), 0, s, gitem,
                        work + L.s1, (int)(B * ny), nx);
     cb.z = z;
@@ -2215,7 +2287,7 @@ extern "C" int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z
   rb.screen = 0;
   rb.inverse = 1;
   rb.fwd_items = 0;
-  row(rb, batch, s);
+  run_row(plan, row, rb, batch, s);
   // the weight slice is slice 0 of the volume
   if (!simple)
     launch_grad_reduce(gd, grad_dn, batch, nn, 1, nullptr, 0.f, s);

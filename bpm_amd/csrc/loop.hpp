@@ -44,7 +44,7 @@
 //   256^2  batch 1: 7.0 (4.4) against 10.1;  8: 7.0 against 13.7;
 //          batch 16: 8.6 against 18.8;       50: 24.8 (8.8) against 37.4
 //   512^2  batch 1: 14.0 (8.8) against 12.5; 2: 14.3 against 15.7;
-//          batch 8: 14.2 against 35.7;       50: 94.9 against 118.5
+//          batch 8: 14.2 against 30.9;       50: 94.9 against 100.6
 // What bounds a phase now: at 64^2 its chain of L2, LDS and flag latencies
 // (2.1 us), at 512^2 the transforms' instruction issue on the XCD's 32 CUs
 // (a field-step of 512^2 on one XCD is about 9 us of issue).

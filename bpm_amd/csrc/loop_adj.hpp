@@ -21,7 +21,7 @@
 //   256^2  batch 1: 8.0 against 12.4,          24.6 against 39.8
 //          batch 8: 8.8 against 18.8,          25.1 against 52.9
 //          batch 50: 37.6 against 54.7,        136 against 173
-//   512^2  batch 8: 34.4 against 38.6,         81 against 120
+//   512^2  batch 8: 34.2 against 34.5,         81 against 116
 // A mean-corrected step is 6 phases (3 of them adjoint) and the float64 sines
 // of its propagator; what bounds a phase is as in loop.hpp.
 #pragma once
