@@ -1176,48 +1176,55 @@ static int items_per(long long threads, int batch) {
   return (batch + chunks - 1) / chunks;
 }
 
-template <int NX>
+template <int NX, int E>
 static void launch_row_items(const RowArgs& a, int batch, hipStream_t s) {
-  constexpr int E = row_e_of(NX, 0), T = NX / E, LINES = T >= 256 ? 1 : 256 / T;
+  constexpr int T = NX / E, LINES = T >= 256 ? 1 : 256 / T, W = E == 4 ? 5 : 3;
   const bool shared = a.ngroups == 0 && a.dn_bstride == 0 && a.dn0_mode != BPMH_MEAN_WEIGHTED;
   const int per = shared || !a.screen ? items_per((long long)batch * a.ny * T, batch) : 1;
   const dim3 g(a.ny / LINES, (batch + per - 1) / per), b(T * LINES);
-  if (a.adjoint) hipLaunchKernelGGL((k_row_items<NX, E, LINES, E == 4 ? 5 : 3, true>), g, b, 0, s, a, batch, per);
-  else hipLaunchKernelGGL((k_row_items<NX, E, LINES, E == 4 ? 5 : 3, false>), g, b, 0, s, a, batch, per);
+  if (a.adjoint) hipLaunchKernelGGL((k_row_items<NX, E, LINES, W, true>), g, b, 0, s, a, batch, per);
+  else hipLaunchKernelGGL((k_row_items<NX, E, LINES, W, false>), g, b, 0, s, a, batch, per);
 }
-template <int NY>
+template <int NY, int E>
 static void launch_col_items(const ColArgs& a, int batch, hipStream_t s) {
-  constexpr int E = col_e_of(NY, 0), T = NY / E, LC = T >= 128 ? 4 : 8;
+  constexpr int T = NY / E, LC = T >= 512 ? 2 : (T >= 128 ? 4 : 8);
   const int per = items_per((long long)batch * a.nx * T, batch);
   const dim3 g(a.nx / LC, (batch + per - 1) / per), b(T * LC);
   if (a.hmode == 0) hipLaunchKernelGGL((k_col_items<NY, E, LC, 4, false>), g, b, 0, s, a, batch, per);
   else hipLaunchKernelGGL((k_col_items<NY, E, LC, 4, true>), g, b, 0, s, a, batch, per);
 }
+template <int N>
+static void run_row_items(int ealt, const RowArgs& a, int batch, hipStream_t s) {
+  if (ealt) launch_row_items<N, row_e_of(N, 1)>(a, batch, s);
+  else launch_row_items<N, row_e_of(N, 0)>(a, batch, s);
+}
+template <int N>
+static void run_col_items(int ealt, const ColArgs& a, int batch, hipStream_t s) {
+  if (ealt) launch_col_items<N, col_e_of(N, 1)>(a, batch, s);
+  else launch_col_items<N, col_e_of(N, 0)>(a, batch, s);
+}
 
+// One row pass of a call; row: the plan's one-item pass.
 static void run_row(bpmh_plan plan, row_fn row, const RowArgs& a, int batch, hipStream_t s) {
-  const int nx = plan->nx;
+  const int nx = plan->nx, ealt = plan->row_v / kRowShapes;
   if ((nx == 512 || nx == 1024 || nx == 2048) && (long long)batch * nx * plan->ny >= kItemsRows &&
       (!a.adjoint || a.screen)) {
-    RowArgs r = a;
-    r.tw = plan->tw_x[0];
-    if (nx == 512) launch_row_items<512>(r, batch, s);
-    else if (nx == 1024) launch_row_items<1024>(r, batch, s);
-    else launch_row_items<2048>(r, batch, s);
+    if (nx == 512) run_row_items<512>(ealt, a, batch, s);
+    else if (nx == 1024) run_row_items<1024>(ealt, a, batch, s);
+    else run_row_items<2048>(ealt, a, batch, s);
   } else {
     row(a, batch, s);
   }
 }
 
-// Column passes with H of a table or of n_eff[z].
+// One column pass with H of a table or of n_eff[z].
 static void run_col(bpmh_plan plan, col_fn col, const ColArgs& a, int batch, hipStream_t s) {
-  const int ny = plan->ny;
+  const int ny = plan->ny, ealt = plan->col_v / kColShapes;
   if ((ny == 512 || ny == 1024 || ny == 2048) && (long long)batch * ny * plan->nx >= kItemsCols &&
       !a.sw) {
-    ColArgs r = a;
-    r.tw = plan->tw_y[0];
-    if (ny == 512) launch_col_items<512>(r, batch, s);
-    else if (ny == 1024) launch_col_items<1024>(r, batch, s);
-    else launch_col_items<2048>(r, batch, s);
+    if (ny == 512) run_col_items<512>(ealt, a, batch, s);
+    else if (ny == 1024) run_col_items<1024>(ealt, a, batch, s);
+    else run_col_items<2048>(ealt, a, batch, s);
   } else {
     col(a, batch, s);
   }

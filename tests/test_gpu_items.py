@@ -19,23 +19,25 @@ def say(*a):
     sys.stdout.flush()
 
 
-def plan_of(nx, ny):
+def plan_of(nx, ny, sched=(1, 1)):
     from bpm_amd import _lib
     from bpm_amd import bpm3d as B
     plan = B.Plan(nx, ny)
-    _lib.call("bpmh_plan_set_variant", plan, 1, 1)
+    _lib.call("bpmh_plan_set_variant", plan, *sched)
     _lib.call("bpmh_plan_set_loop", plan, LAUNCHES)
     return plan
 
 
+# both radix schedules of rows and columns
+@pytest.mark.parametrize("sched", [(1, 1), (4, 6)])
 @pytest.mark.parametrize("nx,ny,b", [(512, 512, 9), (1024, 512, 4), (512, 1024, 37), (2048, 512, 3),
                                      (256, 2048, 5), (1024, 256, 9), (512, 64, 65)])
-def test_items_equal_single_fields(nx, ny, b):
+def test_items_equal_single_fields(nx, ny, b, sched):
     import torch
     from bpm_amd import _lib
     from bpm_amd import bpm3d as B
     assert b * nx * ny >= LIMIT > nx * ny
-    plan = plan_of(nx, ny)
+    plan = plan_of(nx, ny, sched)
     H = B.propagator_table(nx, ny, UNITS, LAM, N0, _lib.H_F64)
     rng = np.random.default_rng(nx + ny + b)
     nz = 3
