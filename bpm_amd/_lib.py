@@ -143,7 +143,32 @@ def to_device(x, np_dtype):
     a = np.ascontiguousarray(np.asarray(x).astype(np_dtype, copy=False))
     if not a.flags.writeable:  # torch.from_numpy wants a writable array
         a = a.copy()
-    return t.from_numpy(a).to(device())
+    return _upload(t.from_numpy(a))
+
+
+def _upload(src):
+    """A contiguous host tensor on the GPU, staged as in to_numpy."""
+    t = torch()
+    dev = device()
+    n = src.numel()
+    if n * src.element_size() <= _STAGE_UP or src.is_pinned():
+        return src.to(dev)
+    out = t.empty(src.shape, dtype=src.dtype, device=dev)
+    flat, dst = src.reshape(-1), out.reshape(-1)
+    with t.cuda.device(out.device):
+        half = _halves(n, src.dtype)
+        per = half[0].numel()
+        stream = t.cuda.current_stream()
+        done = [None, None]
+        for i in range((n + per - 1) // per):
+            part = flat[i * per:(i + 1) * per]
+            if done[i & 1] is not None:
+                done[i & 1].synchronize()
+            half[i & 1][:part.numel()].copy_(part)
+            dst[i * per:(i + 1) * per].copy_(half[i & 1][:part.numel()], non_blocking=True)
+            done[i & 1] = t.cuda.Event()
+            done[i & 1].record(stream)
+    return out
 
 
 def empty(shape, np_dtype):
@@ -166,5 +191,53 @@ def is_tensor(x):
     return isinstance(x, t.Tensor)
 
 
+# Bytes of each half of the pinned staging memory of a copy between host arrays
+# and the GPU.  A copy that HIP stages itself moves 4 GB/s to the host (53 MB:
+# 12.2 ms); through pinned halves, one filled by the copy engine while all host
+# threads empty the other into a fresh numpy array (whose large pages numpy asks
+# for), it moves 46 GB/s (1.1 ms; halves of 1 MiB 4.4, 4 MiB 2.3).  Uploads:
+# 1.8 against 1.1 ms.  Below _STAGE_DOWN and _STAGE_UP staging costs more than it
+# gives (256 KB down: 44 against 25 us; 2 MB up: 86 against 86).  The memory is
+# torch's pinned pool's: taken for the call and given back.
+_STAGE = 8 << 20
+_STAGE_DOWN, _STAGE_UP = 512 << 10, 2 << 20
+
+
+def _halves(n, dtype):
+    """Pinned staging for n elements: one buffer if they fit, else two halves."""
+    t = torch()
+    per = max(1, _STAGE // t.empty(0, dtype=dtype).element_size())
+    return [t.empty(min(n, per), dtype=dtype, pin_memory=True) for _ in range(1 if n <= per else 2)]
+
+
 def to_numpy(x):
-    return x.cpu().numpy()
+    """The tensor as a numpy array; a GPU tensor is copied once what its stream
+    holds has run."""
+    n = x.numel()
+    if (not x.is_cuda or n * x.element_size() <= _STAGE_DOWN or not x.is_contiguous() or
+            x.requires_grad or x.is_conj()):
+        return x.cpu().numpy()
+    t = torch()
+    src = x.reshape(-1)
+    with t.cuda.device(x.device):
+        half = _halves(n, x.dtype)
+        per = half[0].numel()
+        stream = t.cuda.current_stream()
+        out = np.empty(tuple(x.shape), half[0].numpy().dtype)
+        dst = t.from_numpy(out.reshape(-1))
+        done = [t.cuda.Event(), t.cuda.Event()]
+
+        def fetch(i):
+            part = src[i * per:(i + 1) * per]
+            half[i & 1][:part.numel()].copy_(part, non_blocking=True)
+            done[i & 1].record(stream)
+
+        parts = (n + per - 1) // per
+        fetch(0)
+        for i in range(parts):
+            if i + 1 < parts:
+                fetch(i + 1)
+            done[i & 1].synchronize()
+            part = dst[i * per:(i + 1) * per]
+            part.copy_(half[i & 1][:part.numel()])
+    return out

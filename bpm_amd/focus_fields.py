@@ -178,11 +178,11 @@ def focus_field_debye_gauss(shape, units, lam, NAs, sig=1. / np.sqrt(2), n_integ
 def psf(shape, units, lam, NA, n0=1., n_integration_steps=200, return_field=False):
     """3-D PSF of an aberration-free system via the vectorial Debye integral
     (bpm/psf/psf_functions.py:18-71): u, or (u, ex, ey, ez) if return_field."""
-    u, ex, ey, ez = focus_field_debye(shape=shape, units=units, lam=lam, NA=NA, n0=n0,
-                                      n_integration_steps=n_integration_steps)
     if return_field:
-        return u, ex, ey, ez
-    return u
+        return focus_field_debye(shape=shape, units=units, lam=lam, NA=NA, n0=n0,
+                                 n_integration_steps=n_integration_steps)
+    u = focus_field_debye_device(shape, units, lam, NA, n0, n_integration_steps)[0]
+    return _lib.to_numpy(u)
 
 
 def psf_lightsheet(shape, units, lam_illum, NA_illum, lam_detect, NA_detect, n0=1.,
@@ -201,9 +201,9 @@ def psf_u0(shape, units, zfoc=0, NA=.4, lam=.5, n0=1., n_integration_steps=200):
     Ex of psf((Nx,Ny,4),(dx,dy,zfoc/2)) at its first plane, z = -zfoc."""
     Nx, Ny = shape
     dx, dy = units
-    u, ex, ey, ez = psf((Nx, Ny, 4), (dx, dy, zfoc / 2.), n0=n0, lam=lam, NA=NA,
-                        n_integration_steps=n_integration_steps, return_field=True)
-    return ex[0, ...]
+    ex = focus_field_debye_device((Nx, Ny, 4), (dx, dy, zfoc / 2.), lam, NA, n0,
+                                  n_integration_steps)[1]
+    return _lib.to_numpy(ex[0])  # the other planes and components stay on the GPU
 
 
 def bessel_jn(n, x):
