@@ -39,14 +39,14 @@
 //
 // Measured, us per step against the launches per pass (65 planes, running
 // sum kept; 4.4, 4.8, 8.8: points per thread of rows and columns):
-//   64^2   batch 1: 4.3 (4.4) against 8.5;   batch 50: 4.6 against 9.6
-//   128^2  batch 1: 5.1 (4.4) against 9.6;   batch 50: 7.3 against 16.6
-//   256^2  batch 1: 7.0 (4.4) against 10.1;  8: 7.0 against 13.7;
-//          batch 16: 8.6 against 18.8;       50: 24.8 (8.8) against 37.4
+//   64^2   batch 1: 4.0 (4.4) against 8.5;   batch 50: 4.4 against 9.6
+//   128^2  batch 1: 4.9 (4.4) against 9.6;   batch 50: 7.2 against 16.6
+//   256^2  batch 1: 6.8 (4.4) against 10.1;  8: 6.7 against 13.7;
+//          batch 16: 8.4 against 18.8;       50: 25.1 (8.8) against 37.4
 //   512^2  batch 1: 14.0 (8.8) against 12.5; 2: 14.3 against 15.7;
 //          batch 8: 14.2 against 30.9;       50: 94.9 against 100.6
 // What bounds a phase now: at 64^2 its chain of L2, LDS and flag latencies
-// (2.1 us), at 512^2 the transforms' instruction issue on the XCD's 32 CUs
+// (2.0 us), at 512^2 the transforms' instruction issue on the XCD's 32 CUs
 // (a field-step of 512^2 on one XCD is about 9 us of issue).
 #pragma once
 #include "passes.hpp"
@@ -164,7 +164,8 @@ BPMH_DEV bool loop_wait(const unsigned* flags, int n, unsigned need) {
   return false;
 }
 
-// dn volume (group) and depth of a field.  The group tables are read at
+// dn volume (group) and depth of a field, looked up once per record (15 compares
+// and selects per phase cost 1 to 3 %).  The group tables are read at
 // constant indices: a kernel argument indexed at run time would be copied to
 // scratch memory whole.
 BPMH_DEV int loop_volume(const RowArgs& ra, int field) {
@@ -194,6 +195,7 @@ struct LoopTeam {
   int lead_field, lead_z;
   bool dead;             // a wait gave up
   int M, field, z0, z1;  // members; the field and its planes z0 (done) to z1
+  int volume;            // the field's dn volume
   bool whole, last;      // M == SLOTS; z1 is the field's last plane
 
   // Registers this work-group; false when there is no team for it.
@@ -287,6 +289,7 @@ struct LoopTeam {
     const int nz = loop_nz(call.ra, call.la, field);
     z1 = min(z0 + (whole ? kLoopSteps : kLoopStepsPart), nz - 1);
     last = z1 == nz - 1;
+    volume = __builtin_amdgcn_readfirstlane(loop_volume(call.ra, field));
     return true;
   }
 
@@ -294,6 +297,13 @@ struct LoopTeam {
   // phase of a chunk: the leader saw that before it wrote the record.)
   BPMH_DEV void enter(bool first, unsigned* sh) {
     if (first) return;
+    // To 32 slots every wavefront reads the flags itself: 2 to 4 % a step less
+    // than one wavefront and a barrier (64^2 4.17 -> 4.03 us, 256^2 weighted
+    // 9.9 -> 9.6); at 512^2's 64 slots the reads of 8 wavefronts cost 3 % more.
+    if constexpr (C::SLOTS <= 32) {
+      dead |= !loop_wait(flags, C::SLOTS, at);
+      return;
+    }
     if (threadIdx.x < 64) {
       const bool ok = loop_wait(flags, C::SLOTS, at);
       if (threadIdx.x == 0) sh[0] = ok;
@@ -309,8 +319,9 @@ struct LoopTeam {
       __hip_atomic_store(flags + s, at + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   }
 
-  // A wait gave up (a member of the team stopped): marks this slot's rows of
-  // the plane; the leader ends the team.
+  // A wait gave up (a member of the team stopped): the wavefront marks its part
+  // of this slot's rows of the plane and ends (barriers then count the others);
+  // the leader ends the team.
   BPMH_DEV void give_up(float2* planes) {
     const __amdgpu_buffer_rsrc_t rp = loop_rsrc(planes + (size_t)field * C::POINTS, C::POINTS * 8);
     const float nan = __uint_as_float(0x7fc00000u);
@@ -446,7 +457,7 @@ k_loop(LoopCall) {
     };
     // element index in ra.dn of row q of slot s at the thread's first point
     auto dn_at = [&](const RowArgs& ra, int s, int q, int z, int line, int tr) __attribute__((always_inline)) {
-      return (size_t)loop_volume(ra, field) * ra.dn_bstride + (size_t)z * (NX * NY) +
+      return (size_t)tm.volume * ra.dn_bstride + (size_t)z * (NX * NY) +
              (size_t)((s * C::LR + q * C::LRP + line) * NX + tr);
     };
     auto load_dpre = [&](const RowArgs& ra, int s, int z, int line, int tr) __attribute__((always_inline)) {
