@@ -1064,9 +1064,11 @@ static bool loop_size(bpmh_plan plan) {
 // rows and columns) runs as one launch.  By size: everywhere from 64^2 to
 // 512 x 256 (1.3 to 2.6 times faster, loop.hpp), except batches beyond 16 with
 // 1024-thread groups (512 x 256 at 4.4, batch 50: 83 against 70 us per step);
-// at 512^2, 32 CUs are too few for a field alone (batch 1: 14.0 against 12.5)
-// and only 8.8 fits two groups a CU (batch 2: 14.3 against 15.7; 16: 27.8
-// against 40; at 4.8 and batch 17 52.7 against 49.5).
+// at 512^2, 32 CUs are too few for a field alone (batch 1: 14.0 against 12.5),
+// only 8.8 fits two groups a CU (batch 2: 14.3 against 15.7; 16: 27.8 against
+// 40; at 4.8 and batch 17 52 against 49.5), and eight fields take a round of
+// 14 us, so not when one or two are left over for the last of three or more
+// (batch 17: 40.9 against 39.8, 20: 41.9 against 45.7, 33: 69 against 64).
 static bool loop_wanted(bpmh_plan plan, int batch, int nz, int er, int ec) {
   const int nx = plan->nx, ny = plan->ny;
   if (plan->loop_mode == 1 || nz < 2 || !loop_size(plan)) return false;
@@ -1074,7 +1076,7 @@ static bool loop_wanted(bpmh_plan plan, int batch, int nz, int er, int ec) {
   // fields of the records: 20 bits each for field, plane and sequence
   if (nz >= (1 << 20) || (long long)batch * (nz / kLoopStepsPart + 2) >= (1 << 20)) return false;
   if (plan->loop_mode >= 2) return true;
-  if (nx * ny == 512 * 512) return er == 8 && batch >= 2;
+  if (nx * ny == 512 * 512) return er == 8 && batch >= 2 && (batch <= 16 || (batch - 1) % 8 > 1);
   if (loop_points(nx, ny) == 4096 && ec == 4) return batch <= 16;
   return true;
 }
