@@ -73,9 +73,8 @@ BPMH_DEV SampleParams sample_params(const DwArgs& a, int i_n, int i_t) {
   const float al1 = a.alphas[2 * i_n], al2 = a.alphas[2 * i_n + 1];
   const float dt = f_div(f_sub(al2, al1), (float)a.S - 1.f);
   const float t = f_add(al1, f_mul((float)i_t, dt));
-  double sd, cd;
-  sincos((double)t, &sd, &cd);
-  const float co = (float)cd, si = (float)sd;
+  const float2 cs = sincos_f32_via_f64(t);
+  const float co = cs.x, si = cs.y;
   const float sq = __fsqrt_rn(co);
   float w;
   if (a.variant == BPMH_DW_INDEX) {
@@ -231,7 +230,7 @@ __global__ void __launch_bounds__(256) k_dw_tables(DwArgs a, int total, int ncol
         float2 v = make_float2(0.f, 0.f);
         if (z < a.nz && s < total) {
           const float kz = k_times(a.lam, axis_coord(z, a.nz, a.z1, a.z2));
-          sincosf(kz * sp[q][0], &v.y, &v.x);
+          v = sincos_f32_via_f64(kz * sp[q][0]);
         }
         P[(size_t)s * zp + z] = v;
       }
@@ -264,6 +263,156 @@ __global__ void __launch_bounds__(256) k_dw_tables(DwArgs a, int total, int ncol
     A[plane + o] = f_mul(sp[q][3], j1);
     A[2 * plane + o] = f_mul(sp[q][4], j2);
   }
+}
+
+// ----------------------------------------------------------------------------
+// few planes: tables and sums in one kernel
+// ----------------------------------------------------------------------------
+// The three integrals of column c on plane z: stored (ITAB), or combined into
+// the fields of its lateral point or points.
+template <bool PAIRS, bool ITAB>
+BPMH_DEV void dw_column_out(const DwArgs& a, int ncols, int z, int c, float2 I0, float2 I1, float2 I2) {
+  if constexpr (ITAB) {
+    float2* o = a.itab + ((size_t)z * ncols + c) * 3;
+    o[0] = I0;
+    o[1] = I1;
+    o[2] = I2;
+  } else {
+    int i, j;
+    if (PAIRS) pair_ij(c, i, j);
+    else i = c % a.nx, j = c / a.nx;
+    const size_t plane = (size_t)z * a.nx * a.ny;
+    const float phi1 = (float)atan2((double)axis_coord(j, a.ny, a.y1, a.y2),
+                                    (double)axis_coord(i, a.nx, a.x1, a.x2));
+    combine(a, dw_trig(phi1), I0, I1, I2, plane + (size_t)j * a.nx + i);
+    if (PAIRS && i != j) {
+      const float phi2 = (float)atan2((double)axis_coord(i, a.ny, a.y1, a.y2),
+                                      (double)axis_coord(j, a.nx, a.x1, a.x2));
+      combine(a, dw_trig(phi2), I0, I1, I2, plane + (size_t)i * a.nx + j);
+    }
+  }
+}
+
+// Grids of NZ <= DW_FEW planes and at least DW_FEW_COLS columns.  The matrix form pads them to a tile of 16 and
+// its amplitude table (12 B per sample and column, 83 MB for a 257^2-pair
+// octant) is written and read once for a few multiply-adds an entry.  Here a
+// work-group of G wavefronts takes 64 columns, wavefront g the samples g, g + G,
+// ...: the amplitudes go from registers into the NZ planes' sums, and the G
+// partial sums are added in order through LDS.  The samples' parameters and
+// phases are evaluated once per work-group (in rounds of DW_FEW_S samples).
+// What bounds it is the instruction issue of the Bessel evaluations and, to
+// 256 work-groups, the chain of one (19 us; a wavefront's samples one after
+// another).  us, tables and product against this, 200 steps:
+//   128 x 128 x 4 (2145 columns)   21.4 against 20.4, the call 45.9 against 47
+//   256 x 256 x 4 (8385)           29.9 against 21.8
+//   512 x 512 x 4 (33153)          53.8 against 41.5;  x 6  51.6 against 42.6
+//   1024 x 1024 x 4                187 against 92
+//   1000 x 600 x 4, 300 steps      307 against 139
+// 16 wavefronts a work-group to 512 work-groups, 8 beyond (512 x 512 x 4: 8
+// wavefronts of 80 registers with spills 46.9, 4 wavefronts 48.3).
+// The first ntb work-groups form the azimuth terms (trig).
+constexpr int DW_FEW = 4;
+constexpr int DW_FEW_COLS = 4096;
+constexpr int DW_FEW_S = 256;
+template <bool PAIRS, bool ITAB, int NZ, int G>
+__global__ void __launch_bounds__((64 * G), 4) k_dw_few(DwArgs a, int total, int ncols, int ntb,
+                                                   float4* __restrict__ trig) {
+  if ((int)blockIdx.x < ntb) {
+    const int k = (int)blockIdx.x * 64 * G + (int)threadIdx.x;
+    if (k >= a.nx * a.ny) return;
+    const float phi = (float)atan2((double)axis_coord(k / a.nx, a.ny, a.y1, a.y2),
+                                   (double)axis_coord(k % a.nx, a.nx, a.x1, a.x2));
+    const DwTrig tr = dw_trig(phi);
+    trig[k] = make_float4(tr.c2, tr.s2, tr.cp, tr.sp);
+    return;
+  }
+  __shared__ float4 sp[DW_FEW_S];        // sin t and the three amplitude factors
+  __shared__ float2 ph[DW_FEW_S][NZ];    // e^{i kz cos t}
+  __shared__ float sums[G][64][6 * NZ + 1];
+  const int l = threadIdx.x & 63, g = threadIdx.x >> 6;
+  const int col = ((int)blockIdx.x - ntb) * 64 + l;
+  float kr = 0.f;
+  if (col < ncols) {
+    int i, j;
+    if (PAIRS) pair_ij(col, i, j);
+    else i = col % a.nx, j = col / a.nx;
+    const float x = axis_coord(i, a.nx, a.x1, a.x2);
+    const float y = axis_coord(j, a.ny, a.y1, a.y2);
+    kr = k_times(a.lam, __fsqrt_rn(f_add(f_mul(x, x), f_mul(y, y))));
+  }
+  float acc[NZ][6];
+#pragma unroll
+  for (int z = 0; z < NZ; ++z)
+#pragma unroll
+    for (int n = 0; n < 6; ++n) acc[z][n] = 0.f;
+  for (int s0 = 0; s0 < total; s0 += DW_FEW_S) {
+    const int ns = min(DW_FEW_S, total - s0);
+    __syncthreads();  // the round before is done with the samples
+    // items: the ns samples' parameters, then their phases plane by plane
+    for (int e = threadIdx.x; e < ns * (NZ + 1); e += 64 * G) {
+      const int z = e / ns - 1, k = e - (z + 1) * ns, s = s0 + k;
+      const SampleParams p = sample_params(a, s / (a.S + 1), s % (a.S + 1));
+      if (z < 0) {
+        sp[k] = make_float4(p.si, f_mul(p.w, f_add(p.co, 1.f)), f_mul(p.w, p.si),
+                            f_mul(p.w, f_sub(p.co, 1.f)));
+      } else {
+        const float kz = k_times(a.lam, axis_coord(z, a.nz, a.z1, a.z2));
+        ph[k][z] = sincos_f32_via_f64(kz * p.co);
+      }
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int k = g; k < ns; k += G) {
+      const float4 q = sp[k];
+      float j0, j1, j2;
+      bpmbessel::j012_f32(f_mul(kr, q.x), j0, j1, j2);
+      const float a0 = f_mul(q.y, j0), a1 = f_mul(q.z, j1), a2 = f_mul(q.w, j2);
+#pragma unroll
+      for (int z = 0; z < NZ; ++z) {
+        const float2 e = ph[k][z];
+        acc[z][0] = fmaf(e.x, a0, acc[z][0]);
+        acc[z][1] = fmaf(e.y, a0, acc[z][1]);
+        acc[z][2] = fmaf(e.x, a1, acc[z][2]);
+        acc[z][3] = fmaf(e.y, a1, acc[z][3]);
+        acc[z][4] = fmaf(e.x, a2, acc[z][4]);
+        acc[z][5] = fmaf(e.y, a2, acc[z][5]);
+      }
+    }
+  }
+#pragma unroll
+  for (int z = 0; z < NZ; ++z)
+#pragma unroll
+    for (int n = 0; n < 6; ++n) sums[g][l][6 * z + n] = acc[z][n];
+  __syncthreads();
+  // wavefront z adds plane z's partial sums (NZ <= G)
+  if (g < NZ && col < ncols) {
+    float r[6];
+#pragma unroll
+    for (int n = 0; n < 6; ++n) {
+      r[n] = sums[0][l][6 * g + n];
+#pragma unroll
+      for (int w = 1; w < G; ++w) r[n] += sums[w][l][6 * g + n];
+    }
+    dw_column_out<PAIRS, ITAB>(a, ncols, g, col, make_float2(r[0], r[1]), make_float2(r[2], r[3]),
+                               make_float2(r[4], r[5]));
+  }
+}
+
+template <bool PAIRS, bool ITAB, int G>
+static void launch_dw_few(const DwArgs& a, int total, int ncols, float4* trig, hipStream_t st) {
+  const int ntb = trig ? (a.nx * a.ny + 64 * G - 1) / (64 * G) : 0;
+  const dim3 g(ntb + (ncols + 63) / 64), b(64 * G);
+  switch (a.nz) {
+    case 1: hipLaunchKernelGGL((k_dw_few<PAIRS, ITAB, 1, G>), g, b, 0, st, a, total, ncols, ntb, trig); break;
+    case 2: hipLaunchKernelGGL((k_dw_few<PAIRS, ITAB, 2, G>), g, b, 0, st, a, total, ncols, ntb, trig); break;
+    case 3: hipLaunchKernelGGL((k_dw_few<PAIRS, ITAB, 3, G>), g, b, 0, st, a, total, ncols, ntb, trig); break;
+    default: hipLaunchKernelGGL((k_dw_few<PAIRS, ITAB, DW_FEW, G>), g, b, 0, st, a, total, ncols, ntb, trig);
+  }
+}
+template <bool PAIRS, bool ITAB>
+static void launch_dw_few(const DwArgs& a, int total, int ncols, float4* trig, hipStream_t st) {
+  if (ncols <= 64 * 512) launch_dw_few<PAIRS, ITAB, 16>(a, total, ncols, trig, st);
+  else launch_dw_few<PAIRS, ITAB, 8>(a, total, ncols, trig, st);
 }
 
 // MFMA form of the product (v_mfma_f32_16x16x4f32; wave64 operand layout:
@@ -883,7 +1032,8 @@ static int debye_grid_run(DwArgs& a, int int_steps, int n_alphas, hipStream_t st
   const int tp = (total + 15) / 16 * 16;
   const int nzt = (nz + 15) / 16, zp = nzt * 16;
   const int cp = (ntab + 16 * DM_CT - 1) / (16 * DM_CT) * (16 * DM_CT);
-  const size_t nA = (size_t)3 * tp * cp, nP = (size_t)tp * zp;
+  const bool few = nz <= DW_FEW && ntab >= DW_FEW_COLS;  // no tables
+  const size_t nA = few ? 0 : (size_t)3 * tp * cp, nP = few ? 0 : (size_t)tp * zp;
   // the product's one-dimensional grid: column blocks x plane groups, padded
   // to a multiple of 8 XCDs
   const int wpg = dw_waves_per_group(nzt);
@@ -923,7 +1073,15 @@ static int debye_grid_run(DwArgs& a, int int_steps, int n_alphas, hipStream_t st
     a.ez = oex + 2 * noct;
     a.I = (float*)(oex + 3 * noct);
   }
-  int rc = dw_timed(0, st, [&] {
+  int rc = BPMH_OK;
+  if (few) {
+    rc = dw_timed(1, st, [&] {
+      if (itab_path) launch_dw_few<true, true>(a, total, ntab, trig, st);
+      else if (pairs) launch_dw_few<true, false>(a, total, ntab, nullptr, st);
+      else launch_dw_few<false, false>(a, total, ncols, nullptr, st);
+    });
+  } else {
+  rc = dw_timed(0, st, [&] {
     const dim3 tgrid((cp + 255) / 256 + 2, tp / DW_SB);  // tp: a multiple of 16
     if (pairs)
       hipLaunchKernelGGL((k_dw_tables<true, DW_SB>), tgrid, dim3(256), 0, st, a, total, ntab, tp, cp,
@@ -944,6 +1102,7 @@ static int debye_grid_run(DwArgs& a, int int_steps, int n_alphas, hipStream_t st
       hipLaunchKernelGGL((k_dw_mfma<false, false>), mgrid, dim3(64 * wpg), 0, st, a, ncols, nzt, tp,
                          cp, (const float2*)P, (const float*)A);
   });
+  }
   if (!rc && itab_path)
     rc = dw_timed(2, st, [&] {
       launch_spread_pairs(a, full->nx0, full->ny0, full->nz0, a.itab, trig, full->u, full->ex,
