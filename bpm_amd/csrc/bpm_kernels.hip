@@ -171,6 +171,8 @@ k_col(ColArgs a) {
   // (x0 and nx are even)
   float2 v[P][E];
   Twiddles<NY, E> tw;
+  WeightParts wparts;
+  if constexpr (PHASE == 2) weighted_parts_load(a.wpart + (size_t)b * a.nx, a.nx, wparts);
   // split columns: the twiddles first, so waiting for the first column's
   // data (loads complete in issue order) does not wait for the second's
   if constexpr (SPLIT) tw.load(t, a.tw);
@@ -230,7 +232,7 @@ k_col(ColArgs a) {
   float dn0w = 0.f;
   if constexpr (PHASE == 2) {
     __shared__ float dn0_slot[2];
-    dn0w = weighted_dn0_group(a.wpart + (size_t)b * a.nx, a.nx, dn0_slot);
+    dn0w = weighted_dn0_group(a.wpart + (size_t)b * a.nx, a.nx, wparts, dn0_slot);
     if (bx == 0 && threadIdx.x == 0) {
       a.dn0_item[b] = dn0w;
       if (a.rec_c) {

@@ -146,12 +146,38 @@ BPMH_DEV float2 prop_f32_beta(float kx2, float ky2, float a, float dz, float* be
 // broadcast through LDS, and the work-group of tile 0 stores it for the row
 // pass.  The kernel boundary after pass A orders the partials' stores before
 // these loads.
+// The first 1024 partials are loaded before the work-group's plane (loads
+// complete in order: behind the plane's, the sum waited for all of it, and its
+// loop for one partial after another), those past the end as zeros: weighted
+// steps of 1024^2 34.9 -> 31.0 us (batch 1), 243 -> 207 (16), of 2048^2 123 ->
+// 114.  (Pass A's weight slice loaded before its transform likewise: 193 at
+// batch 16, but 2048^2 121 and 512^2 18.6 -> 19.3, so it is read after it.)
+struct WeightParts {
+  float2 w[16];
+};
+BPMH_DEV void weighted_parts_load(const float2* wp, int nparts, WeightParts& r) {
+  if (threadIdx.x >= 64) return;
+  const __amdgpu_buffer_rsrc_t rs =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float2*>(wp), (short)0, nparts * 8, 0x00020000);
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    const u2 v = __builtin_amdgcn_raw_buffer_load_b64(rs, (int)threadIdx.x * 8, k * 512, 0);
+    r.w[k] = make_float2(__uint_as_float(v.x), __uint_as_float(v.y));
+  }
+}
 // slot[0] receives dn0, slot[1] the weight sum sum|U| (the adjoint needs it).
-BPMH_DEV float weighted_dn0_group(const float2* __restrict__ wp, int nparts, float* slot) {
+BPMH_DEV float weighted_dn0_group(const float2* __restrict__ wp, int nparts, const WeightParts& r,
+                                  float* slot) {
   if (threadIdx.x < 64) {
     const int lane = threadIdx.x;
     float sd = 0.f, su = 0.f;
-    for (int p = lane; p < nparts; p += 64) {
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      sd += r.w[k].x;
+      su += r.w[k].y;
+    }
+    for (int p = 1024 + lane; p < nparts; p += 64) {
       const float2 v = wp[p];
       sd += v.x;
       su += v.y;
