@@ -1070,15 +1070,19 @@ static bool loop_size(bpmh_plan plan) {
 // only 8.8 fits two groups a CU (batch 2: 14.3 against 15.7; 16: 27.8 against
 // 40; at 4.8 and batch 17 52 against 49.5), and eight fields take a round of
 // 14 us, so not when one or two are left over for the last of three or more
-// (batch 17: 40.9 against 39.8, 20: 41.9 against 45.7, 33: 69 against 64).
-static bool loop_wanted(bpmh_plan plan, int batch, int nz, int er, int ec) {
+// (batch 17: 40.9 against 39.8, 20: 41.9 against 45.7, 33: 69 against 64); with
+// the weighted mean's registers a round takes 23.5 us, so it stops at four
+// (batch 32: 94 against 96, 40: 117 against 116, 64: 188 against 169).
+static bool loop_wanted(bpmh_plan plan, int mode, int batch, int nz, int er, int ec) {
   const int nx = plan->nx, ny = plan->ny;
   if (plan->loop_mode == 1 || nz < 2 || !loop_size(plan)) return false;
   if (!((er == 4 && ec == 4) || (er == 4 && ec == 8) || (er == 8 && ec == 8))) return false;  // not built
   // fields of the records: 20 bits each for field, plane and sequence
   if (nz >= (1 << 20) || (long long)batch * (nz / kLoopStepsPart + 2) >= (1 << 20)) return false;
   if (plan->loop_mode >= 2) return true;
-  if (nx * ny == 512 * 512) return er == 8 && batch >= 2 && (batch <= 16 || (batch - 1) % 8 > 1);
+  if (nx * ny == 512 * 512)
+    return er == 8 && batch >= 2 && (batch <= 16 || (batch - 1) % 8 > 1) &&
+           (mode != BPMH_MEAN_WEIGHTED || batch <= 32);
   if (loop_points(nx, ny) == 4096 && ec == 4) return batch <= 16;
   return true;
 }
@@ -1094,7 +1098,7 @@ static bool loop_wanted(bpmh_plan plan, int batch, int nz, int er, int ec) {
 // 116, 50: 546 against 591).
 static bool loop_adj_wanted(bpmh_plan plan, int mode, int batch, int nz, int er, int ec) {
   const long long pts = (long long)plan->nx * plan->ny;
-  if (!loop_wanted(plan, batch, nz, er, ec) || plan->nx / er > 64 || nz > 65536) return false;
+  if (!loop_wanted(plan, BPMH_MEAN_IGNORE, batch, nz, er, ec) || plan->nx / er > 64 || nz > 65536) return false;
   if (plan->loop_mode >= 2 || mode != BPMH_MEAN_IGNORE || pts < 512 * 256) return true;
   return batch >= 2 && batch * pts <= 8LL * 512 * 512;
 }
@@ -1107,7 +1111,8 @@ static int loop_run(bpmh_plan plan, int mode, int batch, int nz, const LoopCall&
                     bool adj = false) {
   const int nx = plan->nx, ny = plan->ny;
   const int er = row_e_of(nx, plan->row_v / kRowShapes), ec = col_e_of(ny, plan->col_v / kColShapes);
-  if (!(adj ? loop_adj_wanted(plan, mode, batch, nz, er, ec) : loop_wanted(plan, batch, nz, er, ec)))
+  if (!(adj ? loop_adj_wanted(plan, mode, batch, nz, er, ec)
+            : loop_wanted(plan, mode, batch, nz, er, ec)))
     return 0;
   loop_launch_fn launch = nx == 64    ? (adj ? bpmh_loop_adj_nx64 : bpmh_loop_nx64)
                           : nx == 128 ? (adj ? bpmh_loop_adj_nx128 : bpmh_loop_nx128)
