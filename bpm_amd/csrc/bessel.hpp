@@ -153,7 +153,7 @@ __host__ __device__ inline float sqrt_f32(float x) {
 #endif
 }
 
-// sin and cos of chi = x - pi/4 (14 <= x < 2^31) in float32: chi less its
+// sin and cos of chi = x - pi/4 (14 <= x < 2^30) in float32: chi less its
 // nearest multiple n of pi/2 in float64 (pi/2 in two parts), then the Taylor
 // series on [-pi/4, pi/4] (sin to r^9, cos to r^10, the omitted terms below
 // 2.5e-9) and the quarter turns.
@@ -239,13 +239,31 @@ __host__ __device__ inline void j012_series_f32(float ax, float& j0, float& j1, 
 #endif
 }
 
+// Arguments beyond the float32 expansion's phase reduction (and NaN), out of line.
+struct J012f {
+  float j0, j1, j2;
+};
+__host__ __device__ __noinline__ inline J012f j012_large_f32(float ax) {
+  double d0, d1, d2;
+  j012_abs((double)ax, d0, d1, d2);
+  return J012f{(float)d0, (float)d1, (float)d2};
+}
+
 // J_0, J_1, J_2 of a float32 argument as float32: the float64 power series
 // below 14 (where float32 would lose digits to cancellation), the float32
-// expansion above.
+// expansion above, float64 from 2^30 on.
 __host__ __device__ inline void j012_f32(float x, float& j0, float& j1, float& j2) {
   const float ax = fabsf(x);
-  if (ax < 14.f) j012_series_f32(ax, j0, j1, j2);
-  else j012_asym_f32(ax, j0, j1, j2);
+  if (ax < 14.f) {
+    j012_series_f32(ax, j0, j1, j2);
+  } else if (ax < 1073741824.f) {
+    j012_asym_f32(ax, j0, j1, j2);
+  } else {
+    const J012f r = j012_large_f32(ax);
+    j0 = r.j0;
+    j1 = r.j1;
+    j2 = r.j2;
+  }
   if (x < 0.f) j1 = -j1;
 }
 

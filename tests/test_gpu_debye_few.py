@@ -43,3 +43,17 @@ def test_plane_equals_the_points(shape):
     # the axis may round a coordinate by an ulp: 2^-23 of its distance times k, on the field
     shift = 2 * np.pi * 1.33 / LAM * 2**-23 * 2 * .1 * max(shape)
     assert np.abs(got - ref).max() <= (2 * (steps + 1) * 2**-24 + 2 * shift) * top
+
+
+@pytest.mark.parametrize("edge", [.05, 14., 2.**30])
+def test_bessel_at_the_edges_of_its_branches(edge):
+    """Within 2 ulp of 1 below 14 (float64 rounded), 8 ulp of the amplitude above."""
+    from scipy.special import jv
+    from bpm_amd.focus_fields import bessel_jn
+    e = np.float32(edge)
+    x = np.concatenate([np.nextafter(e, np.float32(0)) - np.spacing(e) * np.arange(64, dtype=np.float32),
+                        e + np.spacing(e) * np.arange(64, dtype=np.float32), -e[None]]).astype(np.float32)
+    ax = np.abs(x).astype(np.float64)
+    bound = np.where(ax < 14, 2 * 2.**-24, 8 * 2.**-24 * np.sqrt(2 / (np.pi * ax)))
+    for n in range(3):
+        assert np.all(np.abs(bessel_jn(n, x).astype(np.float64) - jv(n, x.astype(np.float64))) <= bound), n
