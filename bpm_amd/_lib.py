@@ -147,7 +147,9 @@ def to_device(x, np_dtype):
 
 
 def _upload(src):
-    """A contiguous host tensor on the GPU, staged as in to_numpy."""
+    """A contiguous host tensor on the GPU, staged as in to_numpy.  The copy is
+    complete when this returns, as with the unstaged one: the tensor may next be
+    used on any stream."""
     t = torch()
     dev = device()
     n = src.numel()
@@ -168,6 +170,7 @@ def _upload(src):
             dst[i * per:(i + 1) * per].copy_(half[i & 1][:part.numel()], non_blocking=True)
             done[i & 1] = t.cuda.Event()
             done[i & 1].record(stream)
+        done[i & 1].synchronize()
     return out
 
 

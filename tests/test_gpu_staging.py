@@ -23,3 +23,21 @@ def test_round_trip(dtype):
     x = torch.arange(6 * (1 << 20), dtype=torch.float32, device="cuda").view(6, 1024, 1024)
     for v in (x[1:5], x[2], x[:, :, ::2], x.transpose(0, 1)):
         assert np.array_equal(_lib.to_numpy(v), v.cpu().numpy())
+
+
+@pytest.mark.parametrize("mib", [3, 8, 9, 40])
+def test_upload_is_complete_on_return(mib):
+    """Uploaded behind other work of one stream, read on another without a wait
+    between the two streams."""
+    import torch
+    from bpm_amd import _lib
+    a = np.random.default_rng(mib).random(mib << 18, dtype=np.float32)
+    one, two = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(one):
+        torch.cuda._sleep(20_000_000)
+        x = _lib.to_device(a, np.float32)
+    with torch.cuda.stream(two):
+        y = x.clone()
+    two.synchronize()
+    assert np.array_equal(y.cpu().numpy(), a)
