@@ -875,9 +875,22 @@ extern "C" int bpmh_plan_set_variant(bpmh_plan p, int row_variant, int col_varia
   if (row_variant < 0 || row_variant >= 2 * kRowShapes || col_variant < 0 ||
       col_variant >= 2 * kColShapes)
     return bpmh_set_error(BPMH_ERR_INVALID, "row variants are 0 to 5; column variants 0 to 9");
-  p->row_v = row_variant;
-  p->col_v = col_variant;
+  __atomic_store_n(&p->row_v, row_variant, __ATOMIC_RELAXED);
+  __atomic_store_n(&p->col_v, col_variant, __ATOMIC_RELAXED);
   return BPMH_OK;
+}
+
+// The variants of one call.  A call reads them once and takes its kernels and
+// its twiddle tables from this copy: another host thread may set the plan's
+// while the call enqueues (the plans of a grid size are shared), and kernels
+// of one radix schedule on the tables of the other give wrong fields.
+struct Variant {
+  int row, col;
+  int row_alt() const { return row / kRowShapes; }  // radix schedules, as ealt
+  int col_alt() const { return col / kColShapes; }
+};
+static Variant plan_variant(bpmh_plan p) {
+  return {__atomic_load_n(&p->row_v, __ATOMIC_RELAXED), __atomic_load_n(&p->col_v, __ATOMIC_RELAXED)};
 }
 
 extern "C" int bpmh_plan_get_variant(bpmh_plan p, int* row_variant, int* col_variant,
@@ -886,9 +899,10 @@ extern "C" int bpmh_plan_get_variant(bpmh_plan p, int* row_variant, int* col_var
   if (!p || !row_variant || !col_variant || !lines_per_group || !cols_per_group || !row_elems ||
       !col_elems)
     return bpmh_set_error(BPMH_ERR_INVALID, "null argument");
-  *row_variant = p->row_v;
-  *col_variant = p->col_v;
-  variant_shape(p->nx, p->ny, p->row_v, p->col_v, lines_per_group, cols_per_group, row_elems,
+  const Variant var = plan_variant(p);
+  *row_variant = var.row;
+  *col_variant = var.col;
+  variant_shape(p->nx, p->ny, var.row, var.col, lines_per_group, cols_per_group, row_elems,
                 col_elems);
   return BPMH_OK;
 }
@@ -1107,10 +1121,10 @@ static bool loop_adj_wanted(bpmh_plan plan, int mode, int batch, int nz, int er,
 // one launch.  Returns 1 when done, 0 when this call runs as launches per pass
 // (size, schedule, or a stream that is being captured: the synchronisation
 // buffer must not be replayed), or an error.
-static int loop_run(bpmh_plan plan, int mode, int batch, int nz, const LoopCall& call0, hipStream_t s,
-                    bool adj = false) {
+static int loop_run(bpmh_plan plan, Variant var, int mode, int batch, int nz, const LoopCall& call0,
+                    hipStream_t s, bool adj = false) {
   const int nx = plan->nx, ny = plan->ny;
-  const int er = row_e_of(nx, plan->row_v / kRowShapes), ec = col_e_of(ny, plan->col_v / kColShapes);
+  const int er = row_e_of(nx, var.row_alt()), ec = col_e_of(ny, var.col_alt());
   if (!(adj ? loop_adj_wanted(plan, mode, batch, nz, er, ec)
             : loop_wanted(plan, mode, batch, nz, er, ec)))
     return 0;
@@ -1213,9 +1227,9 @@ static void run_col_items(int ealt, const ColArgs& a, int batch, hipStream_t s) 
   else launch_col_items<N, col_e_of(N, 0)>(a, batch, s);
 }
 
-// One row pass of a call; row: the plan's one-item pass.
-static void run_row(bpmh_plan plan, row_fn row, const RowArgs& a, int batch, hipStream_t s) {
-  const int nx = plan->nx, ealt = plan->row_v / kRowShapes;
+// One row pass of a call; row: its one-item pass.
+static void run_row(bpmh_plan plan, Variant var, row_fn row, const RowArgs& a, int batch, hipStream_t s) {
+  const int nx = plan->nx, ealt = var.row_alt();
   if ((nx == 512 || nx == 1024 || nx == 2048) && (long long)batch * nx * plan->ny >= kItemsRows &&
       (!a.adjoint || a.screen)) {
     if (nx == 512) run_row_items<512>(ealt, a, batch, s);
@@ -1227,8 +1241,8 @@ static void run_row(bpmh_plan plan, row_fn row, const RowArgs& a, int batch, hip
 }
 
 // One column pass with H of a table or of n_eff[z].
-static void run_col(bpmh_plan plan, col_fn col, const ColArgs& a, int batch, hipStream_t s) {
-  const int ny = plan->ny, ealt = plan->col_v / kColShapes;
+static void run_col(bpmh_plan plan, Variant var, col_fn col, const ColArgs& a, int batch, hipStream_t s) {
+  const int ny = plan->ny, ealt = var.col_alt();
   if ((ny == 512 || ny == 1024 || ny == 2048) && (long long)batch * ny * plan->nx >= kItemsCols &&
       !a.sw) {
     if (ny == 512) run_col_items<512>(ealt, a, batch, s);
@@ -1246,8 +1260,9 @@ static int prop_run(bpmh_plan plan, const PropCall& c, const StepScratch& sc, hi
                     bool may_allocate) {
   const int nx = plan->nx, ny = plan->ny;
   const int batch = c.batch, nz = c.nz;
-  const row_fn row = pick_row(nx, plan->row_v);
-  const int cv = col_variant_for(plan->col_v, c.plane);
+  const Variant var = plan_variant(plan);
+  const row_fn row = pick_row(nx, var.row);
+  const int cv = col_variant_for(var.col, c.plane);
   // the simple mean's propagator is evaluated in the column pass (PHASE 5)
   const col_fn col0 =
       c.mean_mode == BPMH_MEAN_SIMPLE ? pick_col<5>(ny, cv) : pick_col<0>(ny, cv);
@@ -1257,7 +1272,7 @@ static int prop_run(bpmh_plan plan, const PropCall& c, const StepScratch& sc, hi
   RowArgs ra;
   memset(&ra, 0, sizeof ra);
   ra.plane = c.plane;
-  ra.tw = plan->tw_x[plan->row_v / kRowShapes];
+  ra.tw = plan->tw_x[var.row_alt()];
   ra.dn = c.dn;
   ra.dn_bstride = c.dn_bstride;
   ra.dn_kind = c.dn_kind;
@@ -1303,7 +1318,7 @@ static int prop_run(bpmh_plan plan, const PropCall& c, const StepScratch& sc, hi
     memset(&call, 0, sizeof call);
     call.ra = ra;
     call.ca = ca;
-    const int rc = loop_run(plan, c.mean_mode, batch, nz, call, s);
+    const int rc = loop_run(plan, var, c.mean_mode, batch, nz, call, s);
     if (rc < 0) return rc;
     if (rc == 1) {
       if (c.out_scat)
@@ -1331,8 +1346,7 @@ static int prop_run(bpmh_plan plan, const PropCall& c, const StepScratch& sc, hi
     put(&nz, sizeof nz);
     put(&c.mean_mode, sizeof c.mean_mode);
     put(&c.out_scat, sizeof c.out_scat);
-    put(&plan->row_v, sizeof plan->row_v);
-    put(&plan->col_v, sizeof plan->col_v);
+    put(&var, sizeof var);
     for (GraphEntry& g : plan->graphs) {
       if (g.key == key) {
         HIP_TRY(hipGraphLaunch(g.exec, user));
@@ -1363,7 +1377,7 @@ static int prop_run(bpmh_plan plan, const PropCall& c, const StepScratch& sc, hi
   ra.inverse = 0;
   ra.screen = 0;
   ra.fwd_items = nz > 1 ? batch : 0;
-  timed(TK_ROW, [&] { run_row(plan, row, ra, batch, s); });
+  timed(TK_ROW, [&] { run_row(plan, var, row, ra, batch, s); });
   ra.acc_init = 0;
   ra.inverse = 1;
   ra.screen = c.dn_kind != BPMH_DN_NONE;
@@ -1373,11 +1387,11 @@ static int prop_run(bpmh_plan plan, const PropCall& c, const StepScratch& sc, hi
       timed(TK_COL_A, [&] { colA(ca, batch, s); });
       timed(TK_COL_B, [&] { colB(ca, batch, s); });
     } else {
-      timed(TK_COL, [&] { run_col(plan, col0, ca, batch, s); });
+      timed(TK_COL, [&] { run_col(plan, var, col0, ca, batch, s); });
     }
     ra.z = z;
     ra.fwd_items = z < nz - 1 ? batch : 0;
-    timed(TK_ROW, [&] { run_row(plan, row, ra, batch, s); });
+    timed(TK_ROW, [&] { run_row(plan, var, row, ra, batch, s); });
   }
   if (c.out_scat) {
     hipLaunchKernelGGL(k_scatter_final, dim3((nz + 63) / 64, batch), dim3(64), 0, s, sc.spart,
@@ -1548,12 +1562,13 @@ extern "C" int bpmh_floor_steps(bpmh_plan plan, int batch, int nz, float* plane_
   if (dn_numel < (long long)nz * nx * ny)
     return bpmh_set_error(BPMH_ERR_INVALID, "dn holds fewer than nz planes");
   float2* plane = (float2*)plane_;
-  const int cv = col_variant_for(plan->col_v, plane);
+  const Variant var = plan_variant(plan);
+  const int cv = col_variant_for(var.col, plane);
   floor_row_fn fr = nullptr;
   floor_col_fn fc = nullptr;
 #define FLOOR_CASE(N)                          \
   case N:                                      \
-    fr = pick_floor_row_n<N>(plan->row_v);     \
+    fr = pick_floor_row_n<N>(var.row);         \
     break;
   switch (nx) { BPMH_SIZES(FLOOR_CASE) }
 #undef FLOOR_CASE
@@ -1629,9 +1644,9 @@ extern "C" int bpmh_propagate(bpmh_plan plan, int batch, int nz, float* plane, c
 // ----------------------------------------------------------------------------
 // The launches per pass of a ragged batch: group g of items[g] fields, depth
 // nzs[g]; events as in bpmh_propagate_groups.
-static int groups_launches(bpmh_plan plan, row_fn row, col_fn col, RowArgs ra, ColArgs ca, int dn_kind, int n_groups,
-                           const int* items, const int* nzs, int total, void** group_done,
-                           hipStream_t s) {
+static int groups_launches(bpmh_plan plan, Variant var, row_fn row, col_fn col, RowArgs ra, ColArgs ca,
+                           int dn_kind, int n_groups, const int* items, const int* nzs, int total,
+                           void** group_done, hipStream_t s) {
   // items still propagating at plane z (and, for the forward transform, past
   // it): a prefix, the groups being in order of non-increasing depth
   auto items_deeper = [&](int z) {
@@ -1651,7 +1666,7 @@ static int groups_launches(bpmh_plan plan, row_fn row, col_fn col, RowArgs ra, C
   ra.inverse = 0;
   ra.screen = 0;
   ra.fwd_items = items_deeper(1);
-  run_row(plan, row, ra, total, s);
+  run_row(plan, var, row, ra, total, s);
   int rc = mark_done(0);
   if (rc) return rc;
   ra.acc_init = 0;
@@ -1660,10 +1675,10 @@ static int groups_launches(bpmh_plan plan, row_fn row, col_fn col, RowArgs ra, C
   for (int z = 1; z < nzs[0]; ++z) {
     const int active = items_deeper(z);
     ca.z = z;
-    run_col(plan, col, ca, active, s);
+    run_col(plan, var, col, ca, active, s);
     ra.z = z;
     ra.fwd_items = items_deeper(z + 1);
-    run_row(plan, row, ra, active, s);
+    run_row(plan, var, row, ra, active, s);
     rc = mark_done(z);
     if (rc) return rc;
   }
@@ -1710,14 +1725,15 @@ extern "C" int bpmh_propagate_groups(bpmh_plan plan, int n_groups, const int* it
   int rc = plan_upload(plan);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
-  const row_fn row = pick_row(nx, plan->row_v);
-  const int cv = col_variant_for(plan->col_v, plane);
+  const Variant var = plan_variant(plan);
+  const row_fn row = pick_row(nx, var.row);
+  const int cv = col_variant_for(var.col, plane);
   const col_fn col = pick_col<0>(ny, cv);
 
   RowArgs ra;
   memset(&ra, 0, sizeof ra);
   ra.plane = plane;
-  ra.tw = plan->tw_x[plan->row_v / kRowShapes];
+  ra.tw = plan->tw_x[var.row_alt()];
   ra.dn = dn;
   ra.dn_bstride = dn_group_stride;
   ra.dn_kind = dn_kind;
@@ -1748,13 +1764,13 @@ extern "C" int bpmh_propagate_groups(bpmh_plan plan, int n_groups, const int* it
   call.ca = ca;
   if (!group_done || n_groups == 1) {
     for (int g = 0; g < n_groups; ++g) call.la.gnz[g] = nzs[g];
-    rc = loop_run(plan, BPMH_MEAN_IGNORE, total, nzs[0], call, s);
+    rc = loop_run(plan, var, BPMH_MEAN_IGNORE, total, nzs[0], call, s);
     if (rc < 0) return rc;
     if (rc == 1) {
       if (group_done && group_done[0]) HIP_TRY(hipEventRecord((hipEvent_t)group_done[0], s));
       return BPMH_OK;
     }
-    return groups_launches(plan, row, col, ra, ca, dn_kind, n_groups, items, nzs, total, group_done, s);
+    return groups_launches(plan, var, row, col, ra, ca, dn_kind, n_groups, items, nzs, total, group_done, s);
   }
   const size_t dn_size = dn_kind == BPMH_DN_F16 ? 2 : (dn_kind == BPMH_DN_C64 ? 8 : 4);
   int g = n_groups;
@@ -1766,7 +1782,7 @@ extern "C" int bpmh_propagate_groups(bpmh_plan plan, int n_groups, const int* it
     call.ra.ngroups = 0;
     call.ra.dn_bstride = 0;
     call.ra.nz = call.ca.nz = nzs[g - 1];
-    rc = loop_run(plan, BPMH_MEAN_IGNORE, items[g - 1], nzs[g - 1], call, s);
+    rc = loop_run(plan, var, BPMH_MEAN_IGNORE, items[g - 1], nzs[g - 1], call, s);
     if (rc < 0) return rc;
     if (rc == 0) break;
     if (group_done[g - 1]) HIP_TRY(hipEventRecord((hipEvent_t)group_done[g - 1], s));
@@ -1774,7 +1790,7 @@ extern "C" int bpmh_propagate_groups(bpmh_plan plan, int n_groups, const int* it
   }
   if (g == 0) return BPMH_OK;
   // the groups left (all of them, unless a synchronisation buffer ran out)
-  return groups_launches(plan, row, col, ra, ca, dn_kind, g, items, nzs, total, group_done, s);
+  return groups_launches(plan, var, row, col, ra, ca, dn_kind, g, items, nzs, total, group_done, s);
 }
 
 // ----------------------------------------------------------------------------
@@ -1934,15 +1950,16 @@ static int adjoint_segment(bpmh_plan plan, int batch, int z_lo, int z_hi, float*
   const int urc = plan_upload(plan);
   if (urc) return urc;
   hipStream_t s = (hipStream_t)stream;
-  const row_fn row = pick_row(nx, plan->row_v);
-  const int cv = col_variant_for(plan->col_v, g);
+  const Variant var = plan_variant(plan);
+  const row_fn row = pick_row(nx, var.row);
+  const int cv = col_variant_for(var.col, g);
   const col_fn col0 = pick_col<0>(ny, cv);
   const int comps = dn_kind == BPMH_DN_C64 ? 2 : 1;  // floats of gradient per voxel
 
   RowArgs ra;
   memset(&ra, 0, sizeof ra);
   ra.plane = g;
-  ra.tw = plan->tw_x[plan->row_v / kRowShapes];
+  ra.tw = plan->tw_x[var.row_alt()];
   ra.dn = dn;
   ra.dn_kind = dn_kind;
   ra.ny = ny;
@@ -1973,7 +1990,7 @@ static int adjoint_segment(bpmh_plan plan, int batch, int z_lo, int z_hi, float*
     call.ra.dn = (const char*)dn + (size_t)z_lo * n * sizeof(float);
     call.ra.nz = nseg;
     call.ca = ca;
-    const int rc = loop_run(plan, BPMH_MEAN_IGNORE, batch, nseg, call, s, true);
+    const int rc = loop_run(plan, var, BPMH_MEAN_IGNORE, batch, nseg, call, s, true);
     if (rc < 0) return rc;
     if (rc == 1) {
       launch_grad_reduce(gitem, grad_dn + (size_t)(z_lo + 1) * n, batch, n, nseg - 1, nullptr, 0.f, s);
@@ -1987,16 +2004,16 @@ static int adjoint_segment(bpmh_plan plan, int batch, int z_lo, int z_hi, float*
     ra.inverse = z != z_hi;
     ra.screen = 1;
     ra.fwd_items = batch;
-    run_row(plan, row, ra, batch, s);
+    run_row(plan, var, row, ra, batch, s);
     launch_grad_reduce(gitem, grad_dn + (size_t)z * n, batch, n, 1, nullptr, 0.f, s);
-    run_col(plan, col0, ca, batch, s);
+    run_col(plan, var, col0, ca, batch, s);
   }
   // back to real space: the gradient with respect to u[z_lo]
   ra.adjoint = 0;
   ra.screen = 0;
   ra.inverse = 1;
   ra.fwd_items = 0;
-  run_row(plan, row, ra, batch, s);
+  run_row(plan, var, row, ra, batch, s);
   HIP_TRY(hipGetLastError());
   return BPMH_OK;
 }
@@ -2014,9 +2031,9 @@ extern "C" int bpmh_adjoint_segment_work(bpmh_plan plan, int batch, int z_lo, in
   if (!plan || !numel) return bpmh_set_error(BPMH_ERR_INVALID, "null argument");
   if (batch < 1 || z_lo < 0 || z_hi < z_lo) return bpmh_set_error(BPMH_ERR_INVALID, "bad range");
   const long long n = (long long)plan->nx * plan->ny * (dn_kind == BPMH_DN_C64 ? 2 : 1);
+  const Variant var = plan_variant(plan);
   const bool loop = loop_adj_wanted(plan, BPMH_MEAN_IGNORE, batch, z_hi - z_lo + 1,
-                                    row_e_of(plan->nx, plan->row_v / kRowShapes),
-                                    col_e_of(plan->ny, plan->col_v / kColShapes));
+                                    row_e_of(plan->nx, var.row_alt()), col_e_of(plan->ny, var.col_alt()));
   *numel = n * batch * (loop ? z_hi - z_lo : 1);
   return BPMH_OK;
 }
@@ -2129,10 +2146,11 @@ extern "C" int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z
   const int urc = plan_upload(plan);
   if (urc) return urc;
   hipStream_t s = (hipStream_t)stream;
-  const row_fn row = pick_row(nx, plan->row_v);
+  const Variant var = plan_variant(plan);
+  const row_fn row = pick_row(nx, var.row);
   float2* plane = (float2*)plane_;
   float2* fp = adjoint ? (float2*)(work + L.fplane) : plane;
-  const int cv = col_variant_for(plan->col_v, fp);
+  const int cv = col_variant_for(var.col, fp);
   const col_fn col0 = simple ? pick_col<5>(ny, cv) : pick_col<0>(ny, cv);
   const col_fn colA = pick_col<1>(ny, cv);
   const col_fn colB = pick_col<2>(ny, cv);
@@ -2147,7 +2165,7 @@ extern "C" int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z
   RowArgs ra;
   memset(&ra, 0, sizeof ra);
   ra.plane = fp;
-  ra.tw = plan->tw_x[plan->row_v / kRowShapes];
+  ra.tw = plan->tw_x[var.row_alt()];
   ra.dn = dn + (size_t)z_lo * n2;
   ra.dn_kind = BPMH_DN_F32;
   ra.ny = ny;
@@ -2191,12 +2209,12 @@ extern "C" int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z
       call.ca.rec_w = work + L.recw;
       call.la.kout_zstride = n2;
     }
-    looped = loop_run(plan, mean_mode, batch, nseg, call, s);
+    looped = loop_run(plan, var, mean_mode, batch, nseg, call, s);
     if (looped < 0) return looped;
   }
   ra.z = 0;
   ra.fwd_items = batch;
-  if (!looped) run_row(plan, row, ra, batch, s);
+  if (!looped) run_row(plan, var, row, ra, batch, s);
   ra.inverse = 1;
   ra.screen = 1;
   for (int z = 1; z < nseg && !looped; ++z) {
@@ -2208,14 +2226,14 @@ extern "C" int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z
       ca.rec_w = work + L.recw + (size_t)(z - 1) * B;
     }
     if (simple) {
-      run_col(plan, col0, ca, batch, s);
+      run_col(plan, var, col0, ca, batch, s);
     } else {
       colA(ca, batch, s);
       colB(ca, batch, s);
     }
     ra.z = z;
     ra.fwd_items = z < nseg - 1 ? batch : 0;
-    run_row(plan, row, ra, batch, s);
+    run_row(plan, var, row, ra, batch, s);
   }
   if (!adjoint) {
     HIP_TRY(hipGetLastError());
@@ -2271,7 +2289,7 @@ extern "C" int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z
     call.ca.uk = kseg;
     call.ca.cz = work + L.recc;
     call.ca.wz = work + L.recw;
-    const int rc = loop_run(plan, mean_mode, batch, nseg, call, s, true);
+    const int rc = loop_run(plan, var, mean_mode, batch, nseg, call, s, true);
     if (rc < 0) return rc;
     if (rc == 1) {
       launch_grad_reduce(gitem, grad_dn + (size_t)(z_lo + 1) * nn, batch, nn, nseg - 1,
@@ -2286,7 +2304,7 @@ extern "C" int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z
     rb.useg_z = z;
     rb.inverse = z != nseg - 1;
     if (!simple) rb.dn0_item = work + L.recc + (size_t)(z - 1) * B;
-    run_row(plan, row, rb, batch, s);
+    run_row(plan, var, row, rb, batch, s);
     hipLaunchKernelGGL(k_row_sums, dim3((unsigned)((B * ny + 3) / 4)), dim3(256), 0, s, gitem,
                        work + L.s1, (int)(B * ny), nx);
     cb.z = z;
@@ -2303,7 +2321,7 @@ extern "C" int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z
   rb.screen = 0;
   rb.inverse = 1;
   rb.fwd_items = 0;
-  run_row(plan, row, rb, batch, s);
+  run_row(plan, var, row, rb, batch, s);
   // the weight slice is slice 0 of the volume
   if (!simple)
     launch_grad_reduce(gd, grad_dn, batch, nn, 1, nullptr, 0.f, s);
