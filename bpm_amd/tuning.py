@@ -38,24 +38,19 @@ def load_cache():
     return _cache
 
 
-_index = (None, {})  # (cache it was made from, {(nx, ny): [(batch, best), ...]})
-
-
 def lookup(nx, ny, batch=1):
     """Cached (row_variant, col_variant) for this grid and batch, else for
-    the nearest cached batch of the same grid, else None."""
-    global _index
+    the nearest cached batch of the same grid, else None.  Read from the cache
+    at each call (4 us at most): a re-tuned or replaced entry counts at once."""
     c = load_cache()
-    if _index[0] is not c or sum(len(v) for v in _index[1].values()) != len(c):
-        grids = {}
-        for k, v in c.items():
-            _, grid, b = k.split(":")
-            grids.setdefault(tuple(int(n) for n in grid.split("x")), []).append((int(b), tuple(v["best"])))
-        _index = (c, grids)
-    same = _index[1].get((nx, ny))
-    if not same:
-        return None
-    return min(same, key=lambda e: (abs(e[0] - batch), e[0]))[1]
+    entry = c.get(_key(nx, ny, batch))
+    if entry is None:
+        grid = ":%dx%d:" % (nx, ny)
+        same = [(abs(int(k.rpartition(":")[2]) - batch), k) for k in c if grid in k]
+        if not same:
+            return None
+        entry = c[min(same)[1]]
+    return tuple(entry["best"])
 
 
 ROW_VARIANTS, COL_VARIANTS = 6, 10  # V + 3*s, V + 5*s (s: radix schedule)
