@@ -108,7 +108,7 @@ def _mean_args(units, lam, n0):
 def _mean_call(mode, plane, z0, z1, dnc, means, consts, absorb, g, grad_dn, work):
     n0, k0, dx, dy, dz, unit_k = consts
     n_eff, dn0 = means if means is not None else (None, None)
-    _lib.call("bpmh_mean_segment", B.get_plan(dnc.shape[2], dnc.shape[1], plane.shape[0]), int(mode),
+    _lib.call("bpmh_mean_segment", B.get_plan(dnc.shape[2], dnc.shape[1]), int(mode),
               int(plane.shape[0]), int(z0), int(z1), _lib.ptr(plane), _lib.ptr(dnc),
               int(dnc.numel()), _lib.ptr(n_eff), _lib.ptr(dn0), n0, k0, dx, dy, dz, unit_k,
               int(absorb), _lib.ptr(g) if g is not None else None,
@@ -119,7 +119,7 @@ def _mean_call(mode, plane, z0, z1, dnc, means, consts, absorb, g, grad_dn, work
 def _work(nx, ny, batch, z0, z1, adjoint):
     t = _lib.torch()
     n = ctypes.c_longlong()
-    _lib.call("bpmh_mean_segment_work", B.get_plan(nx, ny, batch), int(batch), int(z0), int(z1),
+    _lib.call("bpmh_mean_segment_work", B.get_plan(nx, ny), int(batch), int(z0), int(z1),
               int(adjoint), ctypes.byref(n))
     return t.empty(int(n.value), dtype=t.float32, device=_lib.device())
 
