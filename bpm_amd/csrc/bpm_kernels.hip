@@ -1008,13 +1008,12 @@ static StepScratch prop_scratch_carve(bpmh_plan plan, const PropCall& c, void* b
 // Synchronisation words of the calls in flight, per device: a call takes a
 // buffer whose last user ran on the same stream (stream order protects it) or
 // has completed, so calls on several streams and host threads never share
-// one.  At most kLoopBufs buffers (each 12 KiB per team and XCD); beyond that
-// a call's stream waits for the buffer used longest ago.  They are freed with
-// the last plan.
+// one.  At most kLoopBufs buffers, each for the largest call (388 KiB), so none
+// is ever replaced while calls are in flight; beyond that a call's stream
+// waits for the buffer used longest ago.  They are freed with the last plan.
 constexpr int kLoopBufs = 16;
 struct LoopBuf {
   unsigned* ptr = nullptr;
-  size_t words = 0;
   hipEvent_t last = nullptr;
   hipStream_t stream = nullptr;
   unsigned long long used = 0;  // 0: never
@@ -1022,14 +1021,14 @@ struct LoopBuf {
 static LoopBuf g_loop_buf[64][kLoopBufs];
 static unsigned long long g_loop_clock = 0;
 
-// Called with g_loop_mu held; -1 and an error when none can be had.
-static int loop_buf_take(int dev, size_t words, hipStream_t s) {
+// Called with g_loop_mu held; -1 when none can be had.
+static int loop_buf_take(int dev, hipStream_t s) {
   LoopBuf* b = g_loop_buf[dev];
   int pick = -1;
   for (int i = 0; i < kLoopBufs && pick < 0; ++i)
-    if (b[i].used && b[i].stream == s && b[i].words >= words) pick = i;
+    if (b[i].used && b[i].stream == s) pick = i;
   for (int i = 0; i < kLoopBufs && pick < 0; ++i)
-    if (!b[i].used || (b[i].words >= words && hipEventQuery(b[i].last) == hipSuccess)) pick = i;
+    if (!b[i].used || hipEventQuery(b[i].last) == hipSuccess) pick = i;
   if (pick < 0) {
     pick = 0;
     for (int i = 1; i < kLoopBufs; ++i)
@@ -1041,20 +1040,11 @@ static int loop_buf_take(int dev, size_t words, hipStream_t s) {
     pick = -1;
   (void)hipGetLastError();  // hipEventQuery's "not ready"
   if (pick < 0) return -1;
-  if (p.words < words) {
-    if (p.used) (void)hipEventSynchronize(p.last);
-    if (p.ptr) (void)hipFree(p.ptr);
-    p.ptr = nullptr;
-    p.words = 0;
-    if (hipMalloc(&p.ptr, words * sizeof(unsigned)) != hipSuccess) {
-      p.ptr = nullptr;
-      (void)hipGetLastError();
-      return -1;
-    }
-    p.words = words;
-  }
-  if (!p.last && hipEventCreateWithFlags(&p.last, hipEventDisableTiming) != hipSuccess) return -1;
-  return pick;
+  if (!p.ptr && hipMalloc(&p.ptr, loop_words(kLoopTeams) * sizeof(unsigned)) != hipSuccess) p.ptr = nullptr;
+  if (!p.last && hipEventCreateWithFlags(&p.last, hipEventDisableTiming) != hipSuccess) p.last = nullptr;
+  if (p.ptr && p.last) return pick;
+  (void)hipGetLastError();
+  return -1;
 }
 
 static void loop_bufs_free() {
@@ -1144,13 +1134,13 @@ static int loop_run(bpmh_plan plan, Variant var, int mode, int batch, int nz, co
   const int slots = loop_slots(nx, ny);
   // teams per XCD: one per field up to what the XCD's 32 CUs hold
   int teams = (batch + 7) / 8;
-  const int most = 256 / slots < 1 ? 1 : 256 / slots;
+  const int most = loop_teams(slots);
   if (teams > most) teams = most;
   call.la.batch = batch;
   call.la.teams = teams;
   const size_t words = loop_words(teams);
   std::lock_guard<std::mutex> lock(g_loop_mu);
-  const int i = loop_buf_take(dev, words, s);
+  const int i = loop_buf_take(dev, s);
   if (i < 0) return 0;
   LoopBuf& b = g_loop_buf[dev][i];
   call.la.sync = b.ptr;
@@ -1160,6 +1150,7 @@ static int loop_run(bpmh_plan plan, Variant var, int mode, int batch, int nz, co
   const bool ok = launch(ny, er, ec, mode, call, plan->loop_mode == 3 ? groups / 4 : groups, s);
   const hipError_t le = hipGetLastError();
   const hipError_t re = hipEventRecord(b.last, s);
+  if (re != hipSuccess) (void)hipStreamSynchronize(s);  // no event tells when the buffer is free
   b.stream = s;
   b.used = ++g_loop_clock;
   if (!ok) return 0;

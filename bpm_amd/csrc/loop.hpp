@@ -67,6 +67,10 @@ constexpr int loop_points(int nx, int ny) {
   return p < 512 ? 512 : (p > 4096 ? 4096 : p);
 }
 constexpr int loop_slots(int nx, int ny) { return nx * ny / loop_points(nx, ny); }
+// Teams per XCD of `slots` members: what its 32 CUs hold of the smallest
+// members (two wavefronts), at most kLoopTeams.
+constexpr int loop_teams(int slots) { return 256 / slots < 1 ? 1 : 256 / slots; }
+constexpr int kLoopTeams = loop_teams(loop_slots(64, 64));
 // 32-bit words of synchronisation state for `teams` teams per XCD
 constexpr size_t loop_words(int teams) {
   return (size_t)kLoopHead + (size_t)kLoopXcds * teams * kLoopTeamWords;
