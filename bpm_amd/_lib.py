@@ -35,6 +35,7 @@ SIGNATURES = {
     "bpmh_plan_kernel_times": (_I, [_P, _P, _P]),
     "bpmh_plan_set_graph": (_I, [_P, _I]),
     "bpmh_plan_set_loop": (_I, [_P, _I]),
+    "bpmh_loop_check": (_I, []),
     "bpmh_plan_set_variant": (_I, [_P, _I, _I]),
     "bpmh_plan_get_variant": (_I, [_P, _P, _P, _P, _P, _P, _P]),
     "bpmh_propagator_table": (_I, [_I, _I, _I, _D, _D, _D, _D, _D, _P, _P]),
@@ -215,7 +216,14 @@ def _halves(n, dtype):
 
 def to_numpy(x):
     """The tensor as a numpy array; a GPU tensor is copied once what its stream
-    holds has run."""
+    holds has run (an error if a z-loop before it gave up)."""
+    out = _to_numpy(x)
+    if x.is_cuda:
+        call("bpmh_loop_check")
+    return out
+
+
+def _to_numpy(x):
     n = x.numel()
     if (not x.is_cuda or n * x.element_size() <= _STAGE_DOWN or not x.is_contiguous() or
             x.requires_grad or x.is_conj()):

@@ -1017,8 +1017,12 @@ struct LoopBuf {
   hipEvent_t last = nullptr;
   hipStream_t stream = nullptr;
   unsigned long long used = 0;  // 0: never
+  unsigned calls = 0;
+  bool zero = false;            // the words are zero, once what is enqueued has run
 };
 static LoopBuf g_loop_buf[64][kLoopBufs];
+// per device, in host memory: set by a call whose waits gave up
+static unsigned* g_loop_failed[64];
 static unsigned long long g_loop_clock = 0;
 
 // Called with g_loop_mu held; -1 when none can be had.
@@ -1055,11 +1059,63 @@ static void loop_bufs_free() {
       if (b.last) (void)hipEventDestroy(b.last);
       b = LoopBuf();
     }
+  for (unsigned*& w : g_loop_failed) {
+    if (w) (void)hipHostFree(w);
+    w = nullptr;
+  }
+}
+
+// Reports, once, that a one-launch call on the device gave up (g_loop_mu held).
+static int loop_failure(int dev) {
+  if (dev < 0 || dev >= 64 || !g_loop_failed[dev] || !__atomic_exchange_n(g_loop_failed[dev], 0u, __ATOMIC_RELAXED))
+    return BPMH_OK;
+  return bpmh_set_error(BPMH_ERR_HIP,
+                        "an earlier one-launch z-loop gave up waiting for its work-groups; its results are NaN");
+}
+
+extern "C" int bpmh_loop_check(void) {
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess) return BPMH_OK;
+  std::lock_guard<std::mutex> lock(g_loop_mu);
+  return loop_failure(dev);
 }
 
 __global__ void k_fill_zero(float* __restrict__ p, size_t n) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0.f;
+}
+
+// After every one-launch call: its synchronisation words are zero again for the
+// next one, and if one of its waits gave up all that it writes becomes NaN and
+// the host's word is set.
+constexpr int kLoopOuts = 9;
+struct LoopDone {
+  unsigned* sync;
+  size_t words;
+  unsigned call;
+  unsigned* failed;
+  float* out[kLoopOuts];  // null: not written by this call
+  size_t n[kLoopOuts];
+};
+__global__ void k_loop_done(LoopDone d) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x, step = (size_t)gridDim.x * blockDim.x;
+  if (i < d.words && i != kLoopFailed) d.sync[i] = 0u;
+  if (d.sync[kLoopFailed] != d.call) return;
+#pragma unroll
+  for (int k = 0; k < kLoopOuts; ++k)
+    if (d.out[k])
+      for (size_t j = i; j < d.n[k]; j += step) d.out[k][j] = __uint_as_float(0x7fc00000u);
+  if (i == 0) __hip_atomic_store(d.failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+static LoopDone loop_done(const LoopCall& c, int points, int nz, size_t words, unsigned* failed) {
+  const size_t plane = (size_t)c.la.batch * points, steps = (size_t)c.la.batch * (nz - 1);
+  const size_t comps = c.ra.dn_kind == BPMH_DN_C64 ? 2 : 1;
+  return {c.la.sync, words, c.la.call, failed,
+          {(float*)c.ra.plane, c.ra.acc, (float*)c.ra.out_field, c.ra.out_intens,
+           c.ca.sw ? (float*)c.ca.spart : nullptr, c.ca.gd_item, c.ra.gitem, c.ca.rec_c, c.ca.cg_out},
+          {2 * plane, plane, 2 * plane * nz, plane * nz, 2 * (size_t)c.la.batch * nz * c.ca.nx, plane,
+           steps * points * comps, steps, steps}};
 }
 
 static bool loop_size(bpmh_plan plan) {
@@ -1140,17 +1196,38 @@ static int loop_run(bpmh_plan plan, Variant var, int mode, int batch, int nz, co
   call.la.teams = teams;
   const size_t words = loop_words(teams);
   std::lock_guard<std::mutex> lock(g_loop_mu);
+  const int rc = loop_failure(dev);
+  if (rc) return rc;
+  unsigned*& failed = g_loop_failed[dev];
+  if (!failed) {
+    if (hipHostMalloc((void**)&failed, sizeof(unsigned), hipHostMallocPortable | hipHostMallocMapped) !=
+        hipSuccess) {
+      failed = nullptr;
+      (void)hipGetLastError();
+      return 0;
+    }
+    *failed = 0;
+  }
   const int i = loop_buf_take(dev, s);
   if (i < 0) return 0;
   LoopBuf& b = g_loop_buf[dev][i];
   call.la.sync = b.ptr;
-  hipLaunchKernelGGL(k_fill_zero, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, s, (float*)b.ptr,
-                     words);
+  if (++b.calls == 0) b.calls = 1;
+  call.la.call = b.calls;
+  call.la.polls = plan->loop_mode == 4 ? 0 : kLoopLimit;
+  if (!b.zero) {
+    const size_t all = loop_words(kLoopTeams);
+    hipLaunchKernelGGL(k_fill_zero, dim3((unsigned)((all + 255) / 256)), dim3(256), 0, s, (float*)b.ptr, all);
+  }
   const int groups = 8 * teams * slots;
   const bool ok = launch(ny, er, ec, mode, call, plan->loop_mode == 3 ? groups / 4 : groups, s);
+  if (ok)
+    hipLaunchKernelGGL(k_loop_done, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, s,
+                       loop_done(call, nx * ny, nz, words, failed));
   const hipError_t le = hipGetLastError();
   const hipError_t re = hipEventRecord(b.last, s);
   if (re != hipSuccess) (void)hipStreamSynchronize(s);  // no event tells when the buffer is free
+  b.zero = ok && le == hipSuccess;
   b.stream = s;
   b.used = ++g_loop_clock;
   if (!ok) return 0;
@@ -1161,7 +1238,7 @@ static int loop_run(bpmh_plan plan, Variant var, int mode, int batch, int nz, co
 
 extern "C" int bpmh_plan_set_loop(bpmh_plan p, int mode) {
   if (!p) return bpmh_set_error(BPMH_ERR_INVALID, "null plan");
-  if (mode < 0 || mode > 3) return bpmh_set_error(BPMH_ERR_INVALID, "loop mode is 0 to 3");
+  if (mode < 0 || mode > 4) return bpmh_set_error(BPMH_ERR_INVALID, "loop mode is 0 to 4");
   p->loop_mode = mode;
   return BPMH_OK;
 }

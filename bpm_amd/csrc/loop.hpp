@@ -21,7 +21,9 @@
 // work-group therefore waits only for others that are already running,
 // whatever is resident; no co-residency is assumed and nothing depends on how
 // the dispatcher deals work-groups to XCDs.  The fields are claimed from one
-// counter by the leaders, deepest first.
+// counter by the leaders, deepest first.  Every wait is bounded: should one give
+// up, the kernel after this one (which clears the synchronisation words, as a
+// kernel before it would) turns the call's results into NaN and tells the host.
 //
 // Memory.  Within an XCD the L2 is the point where all its CUs' accesses
 // meet: stores are written through the CU's L1 to it, and loads with the sc1
@@ -57,8 +59,9 @@ constexpr int kLoopSteps = 64;      // z-steps per record
 constexpr int kLoopStepsPart = 4;   // the same while the team is not complete
 constexpr int kLoopXcds = 16;       // XCD numbers are 4 bits
 constexpr int kLoopTeamWords = 192; // 128 flags, the record, padding
-constexpr int kLoopHead = 64 + 64 * kLoopXcds;  // claim counter, registrations
-constexpr int kLoopLimit = 1 << 25; // polls after which a wait gives up (> 10 s)
+constexpr int kLoopHead = 64 + 64 * kLoopXcds;  // claim counter, failure, registrations
+constexpr int kLoopFailed = 1;  // word: number of the last call a wait of which gave up
+constexpr unsigned kLoopLimit = 1u << 25;  // polls after which a wait gives up (> 10 s)
 
 // Points of a slot: a 32nd of the plane (one slot per CU of an XCD), at least
 // 512 (two wavefronts of 4-point threads) and at most 4096 (1024 threads).
@@ -77,11 +80,13 @@ constexpr size_t loop_words(int teams) {
 }
 
 struct LoopArgs {
-  unsigned* sync;               // loop_words(teams) words, zero at launch
+  unsigned* sync;               // loop_words(teams) words, zero at launch (but kLoopFailed)
   int batch;                    // fields
   int teams;                    // teams per XCD
   int gnz[BPMH_MAX_GROUPS];     // planes of each group of a ragged batch
   long long kout_zstride;       // recorded forward: between two steps' k-space planes
+  unsigned call;                // number of this call on `sync`, from 1
+  unsigned polls;               // kLoopLimit; 0 (for tests): every wait gives up
 };
 
 // The kernel's one argument.  It is read through the kernel-argument segment
@@ -153,19 +158,22 @@ BPMH_DEV unsigned long long loop_pack(unsigned seq, bool end, int mlog, int fiel
          ((unsigned long long)mlog << 40) | ((unsigned long long)field << 20) | (unsigned)z;
 }
 
-// One wavefront waits until the n flags are all at least `need`.
+// One wavefront waits until the n flags are all at least `need`.  (The limit is
+// read beside the first poll: before it, it cost 0.5 % at 256^2, 1.6 % in the
+// weighted gradient.)
 BPMH_DEV bool loop_wait(const unsigned* flags, int n, unsigned need) {
   const __amdgpu_buffer_rsrc_t r = loop_rsrc(flags, 128 * 4);
   const int lane = loop_opaque(threadIdx.x & 63);
-  for (int k = 0; k < kLoopLimit; ++k) {
+  const unsigned polls = loop_args().la.polls;
+  for (unsigned k = 0;; ++k) {
     bool ok = true;
     for (int i = lane; i < n; i += 64)
       ok &= __builtin_amdgcn_raw_buffer_load_b32(r, i * 4, 0, kSc1) >= need;
     asm volatile("" ::: "memory");
-    if (__all(ok)) return true;
+    if (__all(ok) && polls != 0) return true;
+    if (k >= polls) return false;
     __builtin_amdgcn_s_sleep(1);
   }
-  return false;
 }
 
 // dn volume (group) and depth of a field, looked up once per record (15 compares
@@ -228,6 +236,7 @@ struct LoopTeam {
   BPMH_DEV void announce() {
     bool end = seq != 0 && !loop_wait(flags, C::SLOTS, at);
     if (threadIdx.x != 0) return;
+    if (end) failed();
     const LoopCall& call = loop_args();
     // the first time, up to ~20 us for the team to come together
     const __amdgpu_buffer_rsrc_t reg = loop_rsrc(call.la.sync, kLoopHead * 4);
@@ -263,7 +272,14 @@ struct LoopTeam {
     if (threadIdx.x < 64) {
       if (me == 0) announce();
       const __amdgpu_buffer_rsrc_t team = loop_rsrc(flags, kLoopTeamWords * 4);
-      for (;;) {
+      for (unsigned k = 0;; ++k) {
+        if (k >= kLoopLimit) {  // the leader stopped
+          if (threadIdx.x == 0) {
+            failed();
+            *sh = 1ull << 43;
+          }
+          break;
+        }
         const loop_u2 w = __builtin_amdgcn_raw_buffer_load_b64(team, 128 * 4, 0, kSc1);
         asm volatile("" ::: "memory");
         const unsigned hi = __builtin_amdgcn_readfirstlane(w.y);
@@ -271,6 +287,7 @@ struct LoopTeam {
         const unsigned s = hi >> 12;
         if (s != seq) {
           seq = s;
+          k = 0;
           if (((hi >> 11) & 1) || me < (1 << ((hi >> 8) & 7))) {
             if (threadIdx.x == 0) *sh = ((unsigned long long)hi << 32) | lo;
             break;
@@ -323,14 +340,15 @@ struct LoopTeam {
       __hip_atomic_store(flags + s, at + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   }
 
-  // A wait gave up (a member of the team stopped): the wavefront marks its part
-  // of this slot's rows of the plane and ends (barriers then count the others);
-  // the leader ends the team.
-  BPMH_DEV void give_up(float2* planes) {
-    const __amdgpu_buffer_rsrc_t rp = loop_rsrc(planes + (size_t)field * C::POINTS, C::POINTS * 8);
-    const float nan = __uint_as_float(0x7fc00000u);
-    for (int i = threadIdx.x; i < C::PTS; i += C::TH)
-      loop_st(rp, i * 8, me * C::PTS * 8, make_float2(nan, nan));
+  // A wait gave up (a member of the team stopped): the kernel after this one
+  // marks what the call wrote.  The wavefront ends (barriers then count the
+  // others), and the leader ends the team.
+  BPMH_DEV void failed() {
+    const LoopArgs& la = loop_args().la;
+    __hip_atomic_store(la.sync + kLoopFailed, la.call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  BPMH_DEV void give_up() {
+    if ((threadIdx.x & 63) == 0) failed();
     if (me == 0 && threadIdx.x == 0) publish(loop_pack(seq + 1, true, 0, 0, 0));
   }
 };
@@ -707,7 +725,7 @@ k_loop(LoopCall) {
       if (!tm.dead) row_phase(z, z == 0);
     }
     if (tm.dead) {
-      tm.give_up(loop_args().ra.plane);
+      tm.give_up();
       return;
     }
   }

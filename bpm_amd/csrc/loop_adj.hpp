@@ -372,7 +372,7 @@ k_loop_adj(LoopCall) {
       if (!tm.dead) row_phase(k, k == 0);
     }
     if (tm.dead) {
-      tm.give_up(loop_args().ra.plane);
+      tm.give_up();
       return;
     }
   }

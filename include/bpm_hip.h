@@ -87,10 +87,17 @@ int bpmh_plan_set_graph(bpmh_plan plan, int enable);
  * launch for the whole z-loop where it measured faster, by grid and batch;
  * 1 always one launch per pass; 2 one launch wherever it is built; 3 as 2
  * with a quarter of its work-groups (what a busy GPU may leave it at first;
- * for tests).  The results are the same bits.  Streams that are being captured, timed plans
- * and bpmh_propagate_noalloc always use one launch per pass.  No reference
- * counterpart. */
+ * for tests); 4 as 2 with waits that give up at once (the results are NaN; for
+ * tests).  The results of 0 to 3 are the same bits.  Streams that are being
+ * captured, timed plans and bpmh_propagate_noalloc always use one launch per
+ * pass.  No reference counterpart. */
 int bpmh_plan_set_loop(bpmh_plan plan, int mode);
+
+/* The one-launch z-loop's waits are bounded (10 s and more).  If one gives up,
+ * because a work-group of the call was stopped, all results of that call are
+ * NaN, and the next call that may use the loop, or this one, returns an error,
+ * once, as soon as the failed call has completed on the current device. */
+int bpmh_loop_check(void);
 
 /* Launch-shape and radix-schedule variants of the row and column passes,
  * chosen per grid size and batch by the autotuner (bpm_amd/tuning.py).
