@@ -1147,6 +1147,28 @@ static bool loop_wanted(bpmh_plan plan, int mode, int batch, int nz, int er, int
   return true;
 }
 
+// us of a step of `fields` fields as one launch and as launches per pass, to
+// about 15 % from 64^2 to 512^2 and 1 to 256 fields (the launches rather too
+// low).  The loop takes rounds of the fields whose teams an XCD holds at once.
+constexpr double kLoopCallUs = 15;  // a loop's start and end
+static double loop_step_us(bpmh_plan plan, int ec, int fields) {
+  const int nx = plan->nx, ny = plan->ny, slots = loop_slots(nx, ny);
+  const int threads = loop_points(nx, ny) / ec;
+  const double pts = (double)nx * ny;
+  int at_once = 32 * (1024 / threads) / slots;
+  if (at_once > loop_teams(slots)) at_once = loop_teams(slots);
+  if (at_once < 1) at_once = 1;
+  auto round = [&](int k) {
+    return (4.2 + 4.1e-5 * pts + 2.5e-5 * pts * (k - 1)) * (threads == 1024 ? 1.3 : 1.);
+  };
+  const int per_xcd = (fields + 7) / 8, full = per_xcd / at_once, rest = per_xcd % at_once;
+  return full * round(at_once) + (rest ? round(rest) : 0.);
+}
+static double launch_step_us(bpmh_plan plan, int fields) {
+  const double v = (double)plan->nx * plan->ny * fields, one = 8.6e-6 * v, many = 5 + 5.9e-6 * v;
+  return 8 + (plan->nx >= 512 && many < one ? many : one);  // (many: passes of several items)
+}
+
 // The same for the adjoint of a segment of nz planes.  Not built for rows of
 // more than one wavefront; the reduction's grid has a block row per plane.
 // Without a mean correction a step is short beside the forward planes it reads
@@ -1710,6 +1732,71 @@ extern "C" int bpmh_propagate(bpmh_plan plan, int batch, int nz, float* plane, c
 // ----------------------------------------------------------------------------
 // ragged batch: groups of fields with their own dn volumes and depths
 // ----------------------------------------------------------------------------
+// How a ragged batch runs as one-launch loops: the number of them, in ends[r]
+// the first (deepest) group of loop r, loop 0 holding the shallowest groups; 0:
+// as launches per pass.  Without events it is one loop.  With events a group's
+// fires at the end of its loop, while the launches, which carry all groups
+// side by side, finish a group after its own depth.  So the groups are cut into
+// the loops that end first among those in which, by the step times above, no
+// group ends later than it would with the launches.  Measured, us until the
+// shallowest / the last group is done: so, as launches, one loop per group:
+//   128^2, 6 jobs of 8 angles x 200 planes   1360 / 1380, 3060 / 3070, 930 / 5450
+//   128^2, 24 x 193, 17 x 150, 9 x 77         400 / 1600, 1240 / 2790, 390 / 2190
+//   256^2, the same                          2310 / 5290, 3180 / 6790, 620 / 5890
+//   256^2, 3 jobs of 1 angle, 200, 150, 100  (launches)   1110 / 2190, 620 / 2740
+//   512^2, 8 x 100, 8 x 80, 8 x 60           2260 / 3900, 3120 / 4530, 930 / 3880
+static int groups_runs(bpmh_plan plan, Variant var, int n, const int* items, const int* nzs, bool events,
+                       int* ends) {
+  const int er = row_e_of(plan->nx, var.row_alt()), ec = col_e_of(plan->ny, var.col_alt());
+  auto wanted = [&](int lo, int hi) {  // groups [lo, hi) as one loop
+    int fields = 0;
+    for (int g = lo; g < hi; ++g) fields += items[g];
+    return loop_wanted(plan, BPMH_MEAN_IGNORE, fields, nzs[lo], er, ec);
+  };
+  if (!events || n == 1) {
+    ends[0] = 0;
+    return wanted(0, n) ? 1 : 0;
+  }
+  int runs = 0;
+  if (plan->loop_mode >= 2) {  // a loop for each depth
+    for (int lo = n, hi = n; lo > 0; hi = lo) {
+      for (--lo; lo > 0 && nzs[lo - 1] == nzs[hi - 1];) --lo;
+      if (!wanted(lo, hi)) return runs;
+      ends[runs++] = lo;
+    }
+    return runs;
+  }
+  // us of the steps that carry groups [lo, hi), and until group g is done
+  // (launches: lo = 0, hi = n)
+  auto until = [&](int lo, int hi, int g, auto&& step) {
+    double us = 0;
+    int fields = 0;
+    for (int k = lo; k < hi; ++k) fields += items[k];
+    for (int k = hi - 1, z = 1; k >= g; fields -= items[k--])
+      if (nzs[k] > z) us += (nzs[k] - z) * step(fields), z = nzs[k];
+    return us;
+  };
+  double best[BPMH_MAX_GROUPS + 1];  // groups [lo, n) done, over their best cut
+  int cut[BPMH_MAX_GROUPS + 1];      // the end of the first group's loop
+  best[n] = 0;
+  for (int lo = n - 1; lo >= 0; --lo) {
+    best[lo] = -1;
+    for (int hi = lo + 1; hi <= n; ++hi) {
+      if (best[hi] < 0 || !wanted(lo, hi)) continue;
+      const double us = best[hi] + kLoopCallUs +
+                        until(lo, hi, lo, [&](int f) { return loop_step_us(plan, ec, f); });
+      const double most = until(0, n, hi - 1, [&](int f) { return launch_step_us(plan, f); });
+      if (us - kLoopCallUs > .95 * most || (best[lo] >= 0 && us >= best[lo])) continue;
+      best[lo] = us;
+      cut[lo] = hi;
+    }
+  }
+  if (best[0] < 0) return 0;
+  for (int lo = 0; lo < n; lo = cut[lo]) ++runs;
+  for (int lo = 0, r = runs; lo < n; lo = cut[lo]) ends[--r] = lo;
+  return runs;
+}
+
 // The launches per pass of a ragged batch: group g of items[g] fields, depth
 // nzs[g]; events as in bpmh_propagate_groups.
 static int groups_launches(bpmh_plan plan, Variant var, row_fn row, col_fn col, RowArgs ra, ColArgs ca,
@@ -1823,42 +1910,39 @@ extern "C" int bpmh_propagate_groups(bpmh_plan plan, int n_groups, const int* it
   ca.hmode = 0;
   ca.H = H;
 
-  // One launch.  Groups that report their completion separately run one after
-  // another, the shallowest first, so that each event fires when its group is
-  // done.
-  LoopCall call;
-  memset(&call, 0, sizeof call);
-  call.ra = ra;
-  call.ca = ca;
-  if (!group_done || n_groups == 1) {
-    for (int g = 0; g < n_groups; ++g) call.la.gnz[g] = nzs[g];
-    rc = loop_run(plan, var, BPMH_MEAN_IGNORE, total, nzs[0], call, s);
-    if (rc < 0) return rc;
-    if (rc == 1) {
-      if (group_done && group_done[0]) HIP_TRY(hipEventRecord((hipEvent_t)group_done[0], s));
-      return BPMH_OK;
-    }
-    return groups_launches(plan, var, row, col, ra, ca, dn_kind, n_groups, items, nzs, total, group_done, s);
-  }
+  // As one-launch loops, each over a run of groups of neighbouring depths, the
+  // shallowest first; all in one without events.
+  int ends[BPMH_MAX_GROUPS];
+  const int runs = groups_runs(plan, var, n_groups, items, nzs, group_done != nullptr, ends);
   const size_t dn_size = dn_kind == BPMH_DN_F16 ? 2 : (dn_kind == BPMH_DN_C64 ? 8 : 4);
-  int g = n_groups;
-  for (int first = total; g > 0; --g) {
-    first -= items[g - 1];
+  int left = n_groups;  // groups [0, left) are still to be run
+  for (int r = 0; r < runs; ++r) {
+    const int lo = ends[r];  // the run is groups [lo, left)
+    int first = 0, fields = 0;
+    for (int g = 0; g < lo; ++g) first += items[g];
+    LoopCall call;
+    memset(&call, 0, sizeof call);
+    call.ra = ra;
+    call.ca = ca;
     call.ra.plane = call.ca.plane = plane + (size_t)first * n;
     call.ra.acc = out_sum ? out_sum + (size_t)first * n : nullptr;
-    if (dn) call.ra.dn = (const char*)dn + (size_t)(g - 1) * dn_group_stride * dn_size;
-    call.ra.ngroups = 0;
-    call.ra.dn_bstride = 0;
-    call.ra.nz = call.ca.nz = nzs[g - 1];
-    rc = loop_run(plan, var, BPMH_MEAN_IGNORE, items[g - 1], nzs[g - 1], call, s);
+    if (dn) call.ra.dn = (const char*)dn + (size_t)lo * dn_group_stride * dn_size;
+    call.ra.ngroups = left - lo;
+    for (int g = lo; g < left; ++g) {
+      call.ra.gend[g - lo] = (fields += items[g]);
+      call.la.gnz[g - lo] = nzs[g];
+    }
+    call.ra.nz = call.ca.nz = nzs[lo];
+    rc = loop_run(plan, var, BPMH_MEAN_IGNORE, fields, nzs[lo], call, s);
     if (rc < 0) return rc;
     if (rc == 0) break;
-    if (group_done[g - 1]) HIP_TRY(hipEventRecord((hipEvent_t)group_done[g - 1], s));
+    for (int g = left - 1; g >= lo && group_done; --g)
+      if (group_done[g]) HIP_TRY(hipEventRecord((hipEvent_t)group_done[g], s));
+    left = lo;
     total = first;
   }
-  if (g == 0) return BPMH_OK;
-  // the groups left (all of them, unless a synchronisation buffer ran out)
-  return groups_launches(plan, var, row, col, ra, ca, dn_kind, g, items, nzs, total, group_done, s);
+  if (left == 0) return BPMH_OK;
+  return groups_launches(plan, var, row, col, ra, ca, dn_kind, left, items, nzs, total, group_done, s);
 }
 
 // ----------------------------------------------------------------------------

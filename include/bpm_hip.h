@@ -207,8 +207,10 @@ int bpmh_propagate_noalloc(bpmh_plan plan, int batch, int nz, float* plane, cons
  * propagating (a prefix of them), so jobs of one grid size but different
  * depths and volumes share one launch sequence; each item gives the bits of
  * bpmh_propagate on its own volume (same plan variant).  group_done: NULL
- * or n_groups HIP events (hipEvent_t) to record on `stream` as soon as that
- * group's planes and sums are final.  dn_numel: elements dn holds (every
+ * or n_groups HIP events (hipEvent_t) to record on `stream` once that group's
+ * planes and sums are final: after its own depth with one launch per pass, at
+ * the end of the loop that carries it where groups run as one-launch loops
+ * (chosen so that no group ends later for it).  dn_numel: elements dn holds (every
  * group's planes must lie inside).  No reference counterpart (the reference
  * propagates one field per call, bpm/bpm/bpm_3d.py:39-101); it serves
  * several requests of one grid size in one launch sequence. */
