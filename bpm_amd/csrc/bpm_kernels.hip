@@ -2224,7 +2224,9 @@ struct WsegLayout {
   size_t wpart, dn0, fplane, useg, kseg, recc, recw, s1, s2, gitem, gd, cg, total;
 };
 
-static WsegLayout wseg_layout(bpmh_plan plan, int batch, int nseg, bool adjoint) {
+// whole: with the screen gradients of every step, which the adjoint as one
+// launch takes; else of one step.
+static WsegLayout wseg_layout(bpmh_plan plan, int batch, int nseg, bool adjoint, bool whole) {
   const int nx = plan->nx, ny = plan->ny;
   WsegLayout L;
   memset(&L, 0, sizeof L);
@@ -2245,8 +2247,7 @@ static WsegLayout wseg_layout(bpmh_plan plan, int batch, int nseg, bool adjoint)
     L.recw = take((S - 1) * B);
     L.s1 = take(B * ny);
     L.s2 = take(B * nx);
-    // screen gradients: of every step where they run as one launch, else of one
-    L.gitem = take(loop_size(plan) ? B * (S - 1) * n2 : B * n2);
+    L.gitem = take(whole ? B * (S - 1) * n2 : B * n2);
     L.gd = take(B * n2);
     L.cg = take(B * S);
   }
@@ -2254,11 +2255,20 @@ static WsegLayout wseg_layout(bpmh_plan plan, int batch, int nseg, bool adjoint)
   return L;
 }
 
+// Whether the adjoint of a mean-corrected segment runs as one launch (of either
+// mean) when its workspace allows.
+static bool wseg_whole(bpmh_plan plan, Variant var, int batch, int nseg) {
+  return loop_adj_wanted(plan, BPMH_MEAN_WEIGHTED, batch, nseg, row_e_of(plan->nx, var.row_alt()),
+                         col_e_of(plan->ny, var.col_alt()));
+}
+
 extern "C" int bpmh_mean_segment_work(bpmh_plan plan, int batch, int z_lo, int z_hi,
                                       int adjoint, long long* numel) {
   if (!plan || !numel) return bpmh_set_error(BPMH_ERR_INVALID, "null argument");
   if (batch < 1 || z_lo < 0 || z_hi < z_lo) return bpmh_set_error(BPMH_ERR_INVALID, "bad range");
-  *numel = (long long)wseg_layout(plan, batch, z_hi - z_lo + 1, adjoint != 0).total;
+  const int nseg = z_hi - z_lo + 1;
+  *numel = (long long)wseg_layout(plan, batch, nseg, adjoint != 0,
+                                  adjoint && wseg_whole(plan, plan_variant(plan), batch, nseg)).total;
   return BPMH_OK;
 }
 
@@ -2288,7 +2298,11 @@ extern "C" int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z
              (long long)(z_hi + 1) * n2);
     return bpmh_set_error(BPMH_ERR_INVALID, msg);
   }
-  const WsegLayout L = wseg_layout(plan, batch, nseg, adjoint);
+  const Variant var = plan_variant(plan);
+  bool whole = adjoint && wseg_whole(plan, var, batch, nseg);
+  // (the workspace may have been asked for at another variant or loop mode)
+  if (whole && work_numel < (long long)wseg_layout(plan, batch, nseg, adjoint, true).total) whole = false;
+  const WsegLayout L = wseg_layout(plan, batch, nseg, adjoint, whole);
   if (work_numel < (long long)L.total) {
     snprintf(msg, sizeof msg, "work holds %lld floats; this segment needs %lld", work_numel,
              (long long)L.total);
@@ -2298,7 +2312,6 @@ extern "C" int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z
   const int urc = plan_upload(plan);
   if (urc) return urc;
   hipStream_t s = (hipStream_t)stream;
-  const Variant var = plan_variant(plan);
   const row_fn row = pick_row(nx, var.row);
   float2* plane = (float2*)plane_;
   float2* fp = adjoint ? (float2*)(work + L.fplane) : plane;
@@ -2432,7 +2445,7 @@ extern "C" int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z
   cb.s2part = work + L.s2;
   cb.s1part = work + L.s1;
   cb.gd_item = gd;
-  {
+  if (whole) {
     LoopCall call;
     memset(&call, 0, sizeof call);
     call.ra = rb;
