@@ -31,7 +31,7 @@ dL/ddn0 / N is added to every voxel of that plane.  Real dn only.
 Memory: checkpoints B*ceil(nz/K) planes + one segment of B*(K+1) planes
 (weighted: about 2*B*(K+2) planes of recorded forward state); where a segment's
 adjoint runs as one launch (grids of 64 to 512 points a side) the screen
-gradients of every step, B*K real planes, instead of B.
+gradients of every step, B*K real planes, instead of B, if they fit the GPU.
 """
 import ctypes
 
@@ -45,6 +45,25 @@ __all__ = ["propagate"]
 
 def _segments(nz, K):
     return [(z0, min(z0 + K, nz - 1)) for z0 in range(0, nz - 1, K)]
+
+
+def _empty(n):
+    return _lib.torch().empty(n, dtype=_lib.torch().float32, device=_lib.device())
+
+
+def _room(full, least, beside=0):
+    """Workspace of `full` floats, or of `least` (with which a segment's adjoint
+    runs as launches per pass) where that, and `beside` floats with it, do not
+    fit the GPU."""
+    if full != least:
+        try:
+            work = _empty(full)
+            _empty(beside)
+            return work
+        except _lib.torch().cuda.OutOfMemoryError:
+            pass
+    work = None
+    return _empty(least)
 
 
 def _make_fn():
@@ -80,9 +99,10 @@ def _make_fn():
             k0dz = float(np.float32(2. * np.pi / lam * units[2]))
             plan = B.get_plan(nx, ny, Bn)
             need = ctypes.c_longlong()
-            _lib.call("bpmh_adjoint_segment_work", plan, int(Bn), 0, max(z1 - z0 for z0, z1 in segs)
-                      if segs else 0, int(kind), ctypes.byref(need))
-            work = t.empty(int(need.value), dtype=t.float32, device=dnc.device)
+            longest = max(z1 - z0 for z0, z1 in segs) if segs else 0
+            _lib.call("bpmh_adjoint_segment_work", plan, int(Bn), 0, longest, int(kind), ctypes.byref(need))
+            least = Bn * ny * nx * (2 if kind == _lib.DN_C64 else 1)
+            work = _room(int(need.value), least, 2 * Bn * (longest + 1) * ny * nx)
             for (z0, z1), ck in zip(reversed(segs), reversed(ckpts)):
                 useg = t.empty((Bn, z1 - z0 + 1, ny, nx), dtype=t.complex64, device=dnc.device)
                 p = ck.clone()
@@ -117,11 +137,12 @@ def _mean_call(mode, plane, z0, z1, dnc, means, consts, absorb, g, grad_dn, work
 
 
 def _work(nx, ny, batch, z0, z1, adjoint):
-    t = _lib.torch()
-    n = ctypes.c_longlong()
-    _lib.call("bpmh_mean_segment_work", B.get_plan(nx, ny), int(batch), int(z0), int(z1),
-              int(adjoint), ctypes.byref(n))
-    return t.empty(int(n.value), dtype=t.float32, device=_lib.device())
+    def need(what):
+        n = ctypes.c_longlong()
+        _lib.call("bpmh_mean_segment_work", B.get_plan(nx, ny), int(batch), int(z0), int(z1), what,
+                  ctypes.byref(n))
+        return int(n.value)
+    return _room(need(1), need(2)) if adjoint else _empty(need(0))
 
 
 def _simple_means(dnc, n0):

@@ -2268,7 +2268,7 @@ extern "C" int bpmh_mean_segment_work(bpmh_plan plan, int batch, int z_lo, int z
   if (batch < 1 || z_lo < 0 || z_hi < z_lo) return bpmh_set_error(BPMH_ERR_INVALID, "bad range");
   const int nseg = z_hi - z_lo + 1;
   *numel = (long long)wseg_layout(plan, batch, nseg, adjoint != 0,
-                                  adjoint && wseg_whole(plan, plan_variant(plan), batch, nseg)).total;
+                                  adjoint == 1 && wseg_whole(plan, plan_variant(plan), batch, nseg)).total;
   return BPMH_OK;
 }
 

@@ -292,7 +292,8 @@ int bpmh_adjoint_segment_ws(bpmh_plan plan, int batch, int z_lo, int z_hi, float
  * work: device floats, at least what bpmh_mean_segment_work reports
  * at the plan's launch shapes (forward: 2*batch*nx + batch; adjoint: about
  * 4*nseg + 4 planes of batch*ny*nx, or 5*nseg where it runs as one launch;
- * with less than that it runs as launches per pass).
+ * with less than that it runs as launches per pass).  adjoint: 0 the forward's
+ * need, 1 the adjoint's, 2 the least that the adjoint takes.
  * Nothing is allocated; calls sharing a work buffer must not overlap.
  * No reference counterpart (the reference has no gradient). */
 int bpmh_mean_segment(bpmh_plan plan, int mean_mode, int batch, int z_lo, int z_hi, float* plane,
