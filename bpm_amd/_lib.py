@@ -154,12 +154,12 @@ def _upload(src):
     t = torch()
     dev = device()
     n = src.numel()
-    if n * src.element_size() <= _STAGE_UP or src.is_pinned():
+    half = None if n * src.element_size() <= _STAGE_UP or src.is_pinned() else _halves(n, src.dtype)
+    if half is None:
         return src.to(dev)
     out = t.empty(src.shape, dtype=src.dtype, device=dev)
     flat, dst = src.reshape(-1), out.reshape(-1)
     with t.cuda.device(out.device):
-        half = _halves(n, src.dtype)
         per = half[0].numel()
         stream = t.cuda.current_stream()
         done = [None, None]
@@ -208,10 +208,14 @@ _STAGE_DOWN, _STAGE_UP = 512 << 10, 2 << 20
 
 
 def _halves(n, dtype):
-    """Pinned staging for n elements: one buffer if they fit, else two halves."""
+    """Pinned staging for n elements: one buffer if they fit, else two halves;
+    None where the host has no memory to pin (the copy is then HIP's own)."""
     t = torch()
     per = max(1, _STAGE // t.empty(0, dtype=dtype).element_size())
-    return [t.empty(min(n, per), dtype=dtype, pin_memory=True) for _ in range(1 if n <= per else 2)]
+    try:
+        return [t.empty(min(n, per), dtype=dtype, pin_memory=True) for _ in range(1 if n <= per else 2)]
+    except RuntimeError:
+        return None
 
 
 def to_numpy(x):
@@ -232,6 +236,8 @@ def _to_numpy(x):
     src = x.reshape(-1)
     with t.cuda.device(x.device):
         half = _halves(n, x.dtype)
+        if half is None:
+            return x.cpu().numpy()
         per = half[0].numel()
         stream = t.cuda.current_stream()
         out = np.empty(tuple(x.shape), half[0].numpy().dtype)

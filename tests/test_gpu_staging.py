@@ -41,3 +41,19 @@ def test_upload_is_complete_on_return(mib):
         y = x.clone()
     two.synchronize()
     assert np.array_equal(y.cpu().numpy(), a)
+
+
+def test_copies_without_pinned_memory(monkeypatch):
+    import torch
+    from bpm_amd import _lib
+    a = np.random.default_rng(1).random(5 << 20, dtype=np.float32)
+    empty = torch.empty
+
+    def none_pinned(*args, pin_memory=False, **kw):
+        if pin_memory:
+            raise RuntimeError("no memory to pin")
+        return empty(*args, **kw)
+
+    monkeypatch.setattr(torch, "empty", none_pinned)
+    x = _lib.to_device(a, np.float32)
+    assert np.array_equal(_lib.to_numpy(x), a)
