@@ -35,6 +35,7 @@ SIGNATURES = {
     "bpmh_plan_kernel_times": (_I, [_P, _P, _P]),
     "bpmh_plan_set_graph": (_I, [_P, _I]),
     "bpmh_plan_set_loop": (_I, [_P, _I]),
+    "bpmh_plan_loop_calls": (_I, [_P, _P]),
     "bpmh_loop_check": (_I, []),
     "bpmh_plan_set_variant": (_I, [_P, _I, _I]),
     "bpmh_plan_get_variant": (_I, [_P, _P, _P, _P, _P, _P, _P]),

@@ -454,6 +454,7 @@ struct bpmh_plan_s {
   std::vector<GraphEntry> graphs;
   unsigned long long graph_clock;
   int loop_mode;                // bpmh_plan_set_loop
+  long long loop_calls;         // z-loops run as one launch
 };
 
 // Wait for an entry's latest replay, then release it.
@@ -574,6 +575,7 @@ extern "C" int bpmh_plan_create(int nx, int ny, bpmh_plan* out) {
   p->cap_stream = nullptr;
   p->graph_clock = 0;
   p->loop_mode = 0;
+  p->loop_calls = 0;
   p->device = -1;
   for (int e = 0; e < 2; ++e) {
     p->tw_x[e] = p->tw_y[e] = nullptr;
@@ -1255,6 +1257,7 @@ static int loop_run(bpmh_plan plan, Variant var, int mode, int batch, int nz, co
   if (!ok) return 0;
   if (le != hipSuccess || re != hipSuccess)
     return bpmh_set_error(BPMH_ERR_HIP, hipGetErrorString(le != hipSuccess ? le : re));
+  ++plan->loop_calls;
   return 1;
 }
 
@@ -1262,6 +1265,13 @@ extern "C" int bpmh_plan_set_loop(bpmh_plan p, int mode) {
   if (!p) return bpmh_set_error(BPMH_ERR_INVALID, "null plan");
   if (mode < 0 || mode > 4) return bpmh_set_error(BPMH_ERR_INVALID, "loop mode is 0 to 4");
   p->loop_mode = mode;
+  return BPMH_OK;
+}
+
+extern "C" int bpmh_plan_loop_calls(bpmh_plan p, long long* calls) {
+  if (!p || !calls) return bpmh_set_error(BPMH_ERR_INVALID, "null argument");
+  std::lock_guard<std::mutex> lock(g_loop_mu);
+  *calls = p->loop_calls;
   return BPMH_OK;
 }
 

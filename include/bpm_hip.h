@@ -92,6 +92,8 @@ int bpmh_plan_set_graph(bpmh_plan plan, int enable);
  * captured, timed plans and bpmh_propagate_noalloc always use one launch per
  * pass.  No reference counterpart. */
 int bpmh_plan_set_loop(bpmh_plan plan, int mode);
+/* z-loops (forward or adjoint) that this plan has enqueued as one launch. */
+int bpmh_plan_loop_calls(bpmh_plan plan, long long* calls);
 
 /* The one-launch z-loop's waits are bounded (10 s and more).  If one gives up,
  * because a work-group of the call was stopped, all results of that call are
