@@ -7,7 +7,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nx,ny", [(512, 256), (256, 512), (512, 64), (64, 512), (512, 128), (128, 128), (256, 256)])
+@pytest.mark.parametrize("nx,ny", [(512, 256), (256, 512), (512, 64), (64, 512), (512, 128), (128, 128), (256, 256), (64, 128), (256, 128)])
 def test_schedules_in_use_are_as_accurate(nx, ny):
     from bpm_amd import bpm3d as B
     from bpm_amd import tuning
@@ -19,6 +19,6 @@ def test_schedules_in_use_are_as_accurate(nx, ny):
         plan.close()
     for v in used:
         print(nx, ny, v, errs[v], flush=True)
-        # (128 points: 4 or 8 are alike, over other inputs the ratio is .96 to 1.05)
+        # (columns of 128 points: 4 or 8 are alike, ratios .92 to 1.05 over ten inputs)
         assert all(e <= 1.05 * f for e, f in zip(errs[v], errs[(1, 1)])), (v, errs)
         assert np.isfinite(errs[v]).all()
