@@ -1238,7 +1238,7 @@ static int loop_run(bpmh_plan plan, Variant var, int mode, int batch, int nz, co
   call.la.sync = b.ptr;
   if (++b.calls == 0) b.calls = 1;
   call.la.call = b.calls;
-  call.la.polls = plan->loop_mode == 4 ? 0 : kLoopLimit;
+  call.la.lost = plan->loop_mode == 4;
   if (!b.zero) {
     const size_t all = loop_words(kLoopTeams);
     hipLaunchKernelGGL(k_fill_zero, dim3((unsigned)((all + 255) / 256)), dim3(256), 0, s, (float*)b.ptr, all);

@@ -86,7 +86,7 @@ struct LoopArgs {
   int gnz[BPMH_MAX_GROUPS];     // planes of each group of a ragged batch
   long long kout_zstride;       // recorded forward: between two steps' k-space planes
   unsigned call;                // number of this call on `sync`, from 1
-  unsigned polls;               // kLoopLimit; 0 (for tests): every wait gives up
+  int lost;                     // tests: every wait gives up (host: which kernel)
 };
 
 // The kernel's one argument.  It is read through the kernel-argument segment
@@ -158,22 +158,23 @@ BPMH_DEV unsigned long long loop_pack(unsigned seq, bool end, int mlog, int fiel
          ((unsigned long long)mlog << 40) | ((unsigned long long)field << 20) | (unsigned)z;
 }
 
-// One wavefront waits until the n flags are all at least `need`.  (The limit is
-// read beside the first poll: before it, it cost 0.5 % at 256^2, 1.6 % in the
-// weighted gradient.)
+// One wavefront waits until the n flags are all at least `need`.  LOST: it gives
+// up at once.  (A template argument: a limit or switch held in a register or
+// read at each wait cost 50 ns of a phase.)
+template <bool LOST>
 BPMH_DEV bool loop_wait(const unsigned* flags, int n, unsigned need) {
+  if constexpr (LOST) return false;
   const __amdgpu_buffer_rsrc_t r = loop_rsrc(flags, 128 * 4);
   const int lane = loop_opaque(threadIdx.x & 63);
-  const unsigned polls = loop_args().la.polls;
-  for (unsigned k = 0;; ++k) {
+  for (unsigned k = 0; k < kLoopLimit; ++k) {
     bool ok = true;
     for (int i = lane; i < n; i += 64)
       ok &= __builtin_amdgcn_raw_buffer_load_b32(r, i * 4, 0, kSc1) >= need;
     asm volatile("" ::: "memory");
-    if (__all(ok) && polls != 0) return true;
-    if (k >= polls) return false;
+    if (__all(ok)) return true;
     __builtin_amdgcn_s_sleep(1);
   }
+  return false;
 }
 
 // dn volume (group) and depth of a field, looked up once per record (15 compares
@@ -197,7 +198,7 @@ BPMH_DEV int loop_nz(const RowArgs& ra, const LoopArgs& la, int field) {
 }
 
 // A work-group's place in its team, and the work that the team is at.
-template <class C>
+template <class C, bool LOST>
 struct LoopTeam {
   unsigned* flags;
   int group, me;
@@ -234,7 +235,7 @@ struct LoopTeam {
 
   // Member 0, one wavefront: the previous chunk is complete, announce the next.
   BPMH_DEV void announce() {
-    bool end = seq != 0 && !loop_wait(flags, C::SLOTS, at);
+    bool end = seq != 0 && !loop_wait<LOST>(flags, C::SLOTS, at);
     if (threadIdx.x != 0) return;
     if (end) failed();
     const LoopCall& call = loop_args();
@@ -322,11 +323,11 @@ struct LoopTeam {
     // than one wavefront and a barrier (64^2 4.17 -> 4.03 us, 256^2 weighted
     // 9.9 -> 9.6); at 512^2's 64 slots the reads of 8 wavefronts cost 3 % more.
     if constexpr (C::SLOTS <= 32) {
-      dead |= !loop_wait(flags, C::SLOTS, at);
+      dead |= !loop_wait<LOST>(flags, C::SLOTS, at);
       return;
     }
     if (threadIdx.x < 64) {
-      const bool ok = loop_wait(flags, C::SLOTS, at);
+      const bool ok = loop_wait<LOST>(flags, C::SLOTS, at);
       if (threadIdx.x == 0) sh[0] = ok;
     }
     __syncthreads();
@@ -420,7 +421,7 @@ BPMH_DEV void loop_screen(const RowArgs& a, int ny, int y, int t, float dn0, con
 }
 
 // MODE: BPMH_MEAN_IGNORE (propagator table), BPMH_MEAN_SIMPLE, BPMH_MEAN_WEIGHTED.
-template <int NX, int NY, int ER, int EC, int MODE>
+template <int NX, int NY, int ER, int EC, int MODE, bool LOST = false>
 __global__ void __launch_bounds__((LoopCfg<NX, NY, ER, EC>::TH), (LoopCfg<NX, NY, ER, EC>::WAVES))
 k_loop(LoopCall) {
   using C = LoopCfg<NX, NY, ER, EC>;
@@ -438,7 +439,7 @@ k_loop(LoopCall) {
   __shared__ float sh_acc[HKEEP ? 1 : C::PTS];  // a complete team's running |u|^2 sums, [element][thread]
   const int tid0 = threadIdx.x;
 
-  LoopTeam<C> tm;
+  LoopTeam<C, LOST> tm;
   if (!tm.join(sh_u)) return;
   {
     const int w = min(loop_args().ra.absorb, HALF);
@@ -739,20 +740,31 @@ bool bpmh_loop_nx128(int, int, int, int, const LoopCall&, int, hipStream_t);
 bool bpmh_loop_nx256(int, int, int, int, const LoopCall&, int, hipStream_t);
 bool bpmh_loop_nx512(int, int, int, int, const LoopCall&, int, hipStream_t);
 
-template <int NX, int NY, int ER, int EC>
-static bool loop_launch_e(int mode, const LoopCall& c, int groups, hipStream_t s) {
+template <int NX, int NY, int ER, int EC, bool LOST>
+static bool loop_launch_m(int mode, const LoopCall& c, int groups, hipStream_t s) {
   const dim3 g((unsigned)groups), b(LoopCfg<NX, NY, ER, EC>::TH);
   switch (mode) {
     case BPMH_MEAN_IGNORE:
-      hipLaunchKernelGGL((k_loop<NX, NY, ER, EC, BPMH_MEAN_IGNORE>), g, b, 0, s, c);
+      hipLaunchKernelGGL((k_loop<NX, NY, ER, EC, BPMH_MEAN_IGNORE, LOST>), g, b, 0, s, c);
       return true;
     case BPMH_MEAN_SIMPLE:
-      hipLaunchKernelGGL((k_loop<NX, NY, ER, EC, BPMH_MEAN_SIMPLE>), g, b, 0, s, c);
+      hipLaunchKernelGGL((k_loop<NX, NY, ER, EC, BPMH_MEAN_SIMPLE, LOST>), g, b, 0, s, c);
       return true;
     case BPMH_MEAN_WEIGHTED:
-      hipLaunchKernelGGL((k_loop<NX, NY, ER, EC, BPMH_MEAN_WEIGHTED>), g, b, 0, s, c);
+      hipLaunchKernelGGL((k_loop<NX, NY, ER, EC, BPMH_MEAN_WEIGHTED, LOST>), g, b, 0, s, c);
       return true;
   }
+  return false;
+}
+
+// the kernels whose waits give up are built for one shape
+template <int NX, int NY, int ER, int EC>
+constexpr bool kLoopLost = NX == 64 && NY == 64 && ER == 4 && EC == 4;
+
+template <int NX, int NY, int ER, int EC>
+static bool loop_launch_e(int mode, const LoopCall& c, int groups, hipStream_t s) {
+  if (!c.la.lost) return loop_launch_m<NX, NY, ER, EC, false>(mode, c, groups, s);
+  if constexpr (kLoopLost<NX, NY, ER, EC>) return loop_launch_m<NX, NY, ER, EC, true>(mode, c, groups, s);
   return false;
 }
 

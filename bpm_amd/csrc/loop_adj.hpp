@@ -52,7 +52,7 @@ BPMH_DEV float loop_row_sum(const float (&w)[E]) {
 // dn at the segment's first plane, nz = the segment's planes, useg, gitem =
 // gvol (nz-1, batch, ny, nx) floats (float2 for complex dn); ca as the column
 // phases 3 and 4 of k_col, uk at the segment's first step.
-template <int NX, int NY, int ER, int EC, int MODE>
+template <int NX, int NY, int ER, int EC, int MODE, bool LOST = false>
 __global__ void __launch_bounds__((LoopCfg<NX, NY, ER, EC>::TH), (LoopCfg<NX, NY, ER, EC>::WAVES))
 k_loop_adj(LoopCall) {
   using C = LoopCfg<NX, NY, ER, EC>;
@@ -71,7 +71,7 @@ k_loop_adj(LoopCall) {
   __shared__ float sh_g[MODE == BPMH_MEAN_WEIGHTED && C::E != 4 ? C::PTS : 1];
   const int tid0 = threadIdx.x;
 
-  LoopTeam<C> tm;
+  LoopTeam<C, LOST> tm;
   if (!tm.join(sh_u)) return;
   {
     const int w = min(loop_args().ra.absorb, HALF);
@@ -383,23 +383,30 @@ bool bpmh_loop_adj_nx128(int, int, int, int, const LoopCall&, int, hipStream_t);
 bool bpmh_loop_adj_nx256(int, int, int, int, const LoopCall&, int, hipStream_t);
 bool bpmh_loop_adj_nx512(int, int, int, int, const LoopCall&, int, hipStream_t);
 
+template <int NX, int NY, int ER, int EC, bool LOST>
+static bool loop_adj_launch_m(int mode, const LoopCall& c, int groups, hipStream_t s) {
+  const dim3 g((unsigned)groups), b(LoopCfg<NX, NY, ER, EC>::TH);
+  switch (mode) {
+    case BPMH_MEAN_IGNORE:
+      hipLaunchKernelGGL((k_loop_adj<NX, NY, ER, EC, BPMH_MEAN_IGNORE, LOST>), g, b, 0, s, c);
+      return true;
+    case BPMH_MEAN_SIMPLE:
+      hipLaunchKernelGGL((k_loop_adj<NX, NY, ER, EC, BPMH_MEAN_SIMPLE, LOST>), g, b, 0, s, c);
+      return true;
+    case BPMH_MEAN_WEIGHTED:
+      hipLaunchKernelGGL((k_loop_adj<NX, NY, ER, EC, BPMH_MEAN_WEIGHTED, LOST>), g, b, 0, s, c);
+      return true;
+  }
+  return false;
+}
+
 template <int NX, int NY, int ER, int EC>
 static bool loop_adj_launch_e(int mode, const LoopCall& c, int groups, hipStream_t s) {
   if constexpr (!LoopCfg<NX, NY, ER, EC>::WAVE) {
     return false;
   } else {
-    const dim3 g((unsigned)groups), b(LoopCfg<NX, NY, ER, EC>::TH);
-    switch (mode) {
-      case BPMH_MEAN_IGNORE:
-        hipLaunchKernelGGL((k_loop_adj<NX, NY, ER, EC, BPMH_MEAN_IGNORE>), g, b, 0, s, c);
-        return true;
-      case BPMH_MEAN_SIMPLE:
-        hipLaunchKernelGGL((k_loop_adj<NX, NY, ER, EC, BPMH_MEAN_SIMPLE>), g, b, 0, s, c);
-        return true;
-      case BPMH_MEAN_WEIGHTED:
-        hipLaunchKernelGGL((k_loop_adj<NX, NY, ER, EC, BPMH_MEAN_WEIGHTED>), g, b, 0, s, c);
-        return true;
-    }
+    if (!c.la.lost) return loop_adj_launch_m<NX, NY, ER, EC, false>(mode, c, groups, s);
+    if constexpr (kLoopLost<NX, NY, ER, EC>) return loop_adj_launch_m<NX, NY, ER, EC, true>(mode, c, groups, s);
     return false;
   }
 }

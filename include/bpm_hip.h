@@ -87,8 +87,8 @@ int bpmh_plan_set_graph(bpmh_plan plan, int enable);
  * launch for the whole z-loop where it measured faster, by grid and batch;
  * 1 always one launch per pass; 2 one launch wherever it is built; 3 as 2
  * with a quarter of its work-groups (what a busy GPU may leave it at first;
- * for tests); 4 as 2 with waits that give up at once (the results are NaN; for
- * tests).  The results of 0 to 3 are the same bits.  Streams that are being
+ * for tests); 4 as 2 with waits that give up at once (the results are NaN; built
+ * for 64^2 points at 4 per thread; for tests).  The results of 0 to 3 are the same bits.  Streams that are being
  * captured, timed plans and bpmh_propagate_noalloc always use one launch per
  * pass.  No reference counterpart. */
 int bpmh_plan_set_loop(bpmh_plan plan, int mode);

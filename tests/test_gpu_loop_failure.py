@@ -1,6 +1,6 @@
-"""Waits of the one-launch z-loop that give up (loop mode 4: no poll counts): every
-kernel ends, all results of the call are NaN, the failure is reported once, and
-the next call is right again."""
+"""Waits of the one-launch z-loop that give up (loop mode 4: at once, whatever the
+flags are): every kernel ends, all results of the call are NaN, the failure is
+reported once, and the next call is right again."""
 import ctypes
 
 import numpy as np
@@ -12,12 +12,12 @@ LAM, N0, UNITS = .5, 1.33, (.1, .1, .1)
 LAUNCHES, LOOP, LOST = 1, 2, 4
 
 
-@pytest.mark.parametrize("nx,ny,b,mode", [(64, 64, 1, "ignore"), (128, 128, 70, "ignore"), (64, 128, 3, "weighted"),
-                                          (512, 512, 2, "ignore")])
-def test_propagation_that_gives_up(nx, ny, b, mode):
+@pytest.mark.parametrize("b,mode", [(1, "ignore"), (300, "ignore"), (3, "weighted")])
+def test_propagation_that_gives_up(b, mode):
     import torch
     from bpm_amd import _lib
     from bpm_amd import bpm3d as B
+    nx = ny = 64
     nz = 5
     rng = np.random.default_rng(4)
     dn = torch.from_numpy(rng.uniform(0, .05, (nz, ny, nx)).astype(np.float32)).cuda()
@@ -41,7 +41,7 @@ def test_propagation_that_gives_up(nx, ny, b, mode):
         return p, acc, vol
 
     try:
-        _lib.call("bpmh_plan_set_variant", plan, *((4, 1) if nx == 512 else (1, 6)))
+        _lib.call("bpmh_plan_set_variant", plan, 1, 6)
         ref = run(LAUNCHES)
         for x in run(LOST):
             assert torch.isnan(torch.view_as_real(x[:b]) if x.is_complex() else x[:b]).all()
@@ -67,7 +67,7 @@ def test_adjoint_that_gives_up(mode):
     import torch
     from bpm_amd import _lib
     from bpm_amd import bpm3d as B
-    nx, ny, b, z_hi = 128, 64, 3, 4
+    nx, ny, b, z_hi = 64, 64, 3, 4
     rng = np.random.default_rng(5)
     cplx = lambda *s: torch.from_numpy((rng.normal(size=s) + 1j * rng.normal(size=s)).astype(np.complex64)).cuda()
     dn = torch.from_numpy(rng.uniform(0, .05, (z_hi + 1, ny, nx)).astype(np.float32)).cuda()
