@@ -136,8 +136,10 @@ _TDT = {np.dtype(np.float32): "float32", np.dtype(np.float16): "float16",
         np.dtype(np.complex64): "complex64"}
 
 
-def to_device(x, np_dtype):
-    """numpy array or torch tensor -> contiguous torch tensor on the GPU with dtype np_dtype."""
+def to_device(x, np_dtype, wait=True):
+    """numpy array or torch tensor -> contiguous torch tensor on the GPU with dtype np_dtype.
+    wait False: for a tensor that the current stream alone uses (a large array's
+    copy may still be under way there)."""
     t = torch()
     tdt = getattr(t, _TDT[np.dtype(np_dtype)])
     if isinstance(x, t.Tensor):
@@ -145,13 +147,13 @@ def to_device(x, np_dtype):
     a = np.ascontiguousarray(np.asarray(x).astype(np_dtype, copy=False))
     if not a.flags.writeable:  # torch.from_numpy wants a writable array
         a = a.copy()
-    return _upload(t.from_numpy(a))
+    return _upload(t.from_numpy(a), wait)
 
 
-def _upload(src):
-    """A contiguous host tensor on the GPU, staged as in to_numpy.  The copy is
-    complete when this returns, as with the unstaged one: the tensor may next be
-    used on any stream."""
+def _upload(src, wait):
+    """A contiguous host tensor on the GPU, staged as in to_numpy.  With wait the
+    copy is complete when this returns, as the unstaged one is: the tensor may
+    next be used on any stream."""
     t = torch()
     dev = device()
     n = src.numel()
@@ -172,7 +174,8 @@ def _upload(src):
             dst[i * per:(i + 1) * per].copy_(half[i & 1][:part.numel()], non_blocking=True)
             done[i & 1] = t.cuda.Event()
             done[i & 1].record(stream)
-        done[i & 1].synchronize()
+        if wait:
+            done[i & 1].synchronize()
     return out
 
 

@@ -297,14 +297,15 @@ def _bpm_3d(size, units, lam=.5, u0=None, dn=None, subsample=1, n0=1.,
         u0 = np.ones((Ny, Nx), np.complex64)
     if tuple(u0.shape) != (Ny, Nx):
         raise ValueError("u0 has shape %s, expected (Ny,Nx)=%s" % (tuple(u0.shape), (Ny, Nx)))
-    plane = _lib.to_device(u0, np.complex64).reshape(1, Ny, Nx).clone()
+    # (this call's stream alone uses both)
+    plane = _lib.to_device(u0, np.complex64, wait=False).reshape(1, Ny, Nx).clone()
 
     kind, ddt = _dn_kind(dn, store_dn_as_half)
     dn_g = None
     if dn is not None:
         if tuple(dn.shape) != (Nz, Ny, Nx):
             raise ValueError("dn has shape %s, expected (Nz,Ny,Nx)=%s" % (tuple(dn.shape), (Nz, Ny, Nx)))
-        dn_g = _lib.to_device(dn, ddt)
+        dn_g = _lib.to_device(dn, ddt, wait=False)
 
     H = n_eff = dn0 = None
     if mean_mode == "ignore":
