@@ -1287,7 +1287,8 @@ extern "C" int bpmh_plan_loop_calls(bpmh_plan p, long long* calls) {
 // Below, their registers leave too few wavefronts to hide a short call's
 // latencies: rows of 2 M points 33.4 against 32.2 (2048 x 64, batch 16), of
 // 1 M 24.3 against 21.7 (1024^2, batch 1); columns of 1 M points 27.9 against
-// 24.9 (256 x 2048, batch 2).
+// 24.9 (256 x 2048, batch 2).  Lines of 512, 1024 and 2048 points have them;
+// there is none for 4096 and shorter lines and the weighted column passes.
 constexpr long long kItemsRows = 5 << 19, kItemsCols = 2 << 20;
 constexpr long long kItemsThreads = 256 << 10;  // 16 wavefronts a CU
 
