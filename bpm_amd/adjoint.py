@@ -47,22 +47,19 @@ def _segments(nz, K):
     return [(z0, min(z0 + K, nz - 1)) for z0 in range(0, nz - 1, K)]
 
 
-def _empty(n):
-    return _lib.torch().empty(n, dtype=_lib.torch().float32, device=_lib.device())
+def _empty(shape, dtype=None):
+    t = _lib.torch()
+    return t.empty(shape, dtype=dtype or t.float32, device=_lib.device())
 
 
-def _room(full, least, beside=0):
+def _room(full, least):
     """Workspace of `full` floats, or of `least` (with which a segment's adjoint
-    runs as launches per pass) where that, and `beside` floats with it, do not
-    fit the GPU."""
-    if full != least:
-        try:
-            work = _empty(full)
-            _empty(beside)
-            return work
-        except _lib.torch().cuda.OutOfMemoryError:
-            pass
-    work = None
+    runs as launches per pass) where that does not fit the GPU."""
+    try:
+        return _empty(full)
+    except _lib.torch().cuda.OutOfMemoryError:
+        if full == least:
+            raise
     return _empty(least)
 
 
@@ -102,9 +99,17 @@ def _make_fn():
             longest = max(z1 - z0 for z0, z1 in segs) if segs else 0
             _lib.call("bpmh_adjoint_segment_work", plan, int(Bn), 0, longest, int(kind), ctypes.byref(need))
             least = Bn * ny * nx * (2 if kind == _lib.DN_C64 else 1)
-            work = _room(int(need.value), least, 2 * Bn * (longest + 1) * ny * nx)
+            work = _room(int(need.value), least)
             for (z0, z1), ck in zip(reversed(segs), reversed(ckpts)):
-                useg = t.empty((Bn, z1 - z0 + 1, ny, nx), dtype=t.complex64, device=dnc.device)
+                shape = (Bn, z1 - z0 + 1, ny, nx)
+                try:
+                    useg = _empty(shape, t.complex64)
+                except t.cuda.OutOfMemoryError:
+                    if work.numel() == least:
+                        raise
+                    work = None
+                if work is None:
+                    work, useg = _empty(least), _empty(shape, t.complex64)
                 p = ck.clone()
                 B.propagate_fields(p, z1 - z0 + 1, units, lam, n0, dn=dnc[z0:],
                                    dn_kind=kind, mean_mode="ignore", H=H,
