@@ -1093,27 +1093,29 @@ __global__ void k_fill_zero(float* __restrict__ p, size_t n) {
 constexpr int kLoopOuts = 9;
 struct LoopDone {
   unsigned* sync;
-  size_t words;
-  unsigned call;
+  unsigned words, call;
   unsigned* failed;
   float* out[kLoopOuts];  // null: not written by this call
   size_t n[kLoopOuts];
 };
-__global__ void k_loop_done(LoopDone d) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x, step = (size_t)gridDim.x * blockDim.x;
+constexpr int kDoneThreads = 256;
+__global__ void __launch_bounds__(kDoneThreads) k_loop_done(LoopDone d) {
+  const unsigned i = blockIdx.x * kDoneThreads + threadIdx.x;
+  const unsigned failed = d.sync[kLoopFailed];  // (under way beside the stores)
   if (i < d.words && i != kLoopFailed) d.sync[i] = 0u;
-  if (d.sync[kLoopFailed] != d.call) return;
+  if (failed != d.call) return;
 #pragma unroll
   for (int k = 0; k < kLoopOuts; ++k)
     if (d.out[k])
-      for (size_t j = i; j < d.n[k]; j += step) d.out[k][j] = __uint_as_float(0x7fc00000u);
+      for (size_t j = i; j < d.n[k]; j += (size_t)gridDim.x * kDoneThreads)
+        d.out[k][j] = __uint_as_float(0x7fc00000u);
   if (i == 0) __hip_atomic_store(d.failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 static LoopDone loop_done(const LoopCall& c, int points, int nz, size_t words, unsigned* failed) {
   const size_t plane = (size_t)c.la.batch * points, steps = (size_t)c.la.batch * (nz - 1);
   const size_t comps = c.ra.dn_kind == BPMH_DN_C64 ? 2 : 1;
-  return {c.la.sync, words, c.la.call, failed,
+  return {c.la.sync, (unsigned)words, c.la.call, failed,
           {(float*)c.ra.plane, c.ra.acc, (float*)c.ra.out_field, c.ra.out_intens,
            c.ca.sw ? (float*)c.ca.spart : nullptr, c.ca.gd_item, c.ra.gitem, c.ca.rec_c, c.ca.cg_out},
           {2 * plane, plane, 2 * plane * nz, plane * nz, 2 * (size_t)c.la.batch * nz * c.ca.nx, plane,
@@ -1246,7 +1248,8 @@ static int loop_run(bpmh_plan plan, Variant var, int mode, int batch, int nz, co
   const int groups = 8 * teams * slots;
   const bool ok = launch(ny, er, ec, mode, call, plan->loop_mode == 3 ? groups / 4 : groups, s);
   if (ok)
-    hipLaunchKernelGGL(k_loop_done, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, s,
+    hipLaunchKernelGGL(k_loop_done, dim3((unsigned)((words + kDoneThreads - 1) / kDoneThreads)),
+                       dim3(kDoneThreads), 0, s,
                        loop_done(call, nx * ny, nz, words, failed));
   const hipError_t le = hipGetLastError();
   const hipError_t re = hipEventRecord(b.last, s);

@@ -60,7 +60,7 @@ constexpr int kLoopStepsPart = 4;   // the same while the team is not complete
 constexpr int kLoopXcds = 16;       // XCD numbers are 4 bits
 constexpr int kLoopTeamWords = 192; // 128 flags, the record, padding
 constexpr int kLoopHead = 64 + 64 * kLoopXcds;  // claim counter, failure, registrations
-constexpr int kLoopFailed = 1;  // word: number of the last call a wait of which gave up
+constexpr int kLoopFailed = 32;  // word (in a line of its own): number of the last call a wait of which gave up
 constexpr unsigned kLoopLimit = 1u << 25;  // polls after which a wait gives up (> 10 s)
 
 // Points of a slot: a 32nd of the plane (one slot per CU of an XCD), at least
